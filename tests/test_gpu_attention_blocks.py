@@ -1,0 +1,61 @@
+"""GPU parity of the attention kernels at the edges of their blocks and variants.
+
+The kernels work in blocks of 128 queries / keys (64 for batches too small to fill
+the chip), 64-token tiles and 32-token halves, and find their (block, row) from the row
+lengths (at most 64 rows) or from the grid (more rows).  Each case puts row ends on
+both sides of those edges, for both block sizes, with and without GQA, and with the
+signs of the softmax scale that the kernels treat apart.
+
+Bar, as in test_gpu_attention.py (fp16 inputs, P and outputs, fp32 sums): against the
+float64 oracle the output within atol = rtol = 2e-3 and the gradients within relative
+L2 1e-2; two calls bit-identical.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import attention as oattn
+from soupsuck_amd.kernels.attention import packed_causal_attention
+
+pytestmark = pytest.mark.gpu
+
+EDGES = (1, 31, 32, 33, 63, 64, 65, 127, 128, 129, 161, 193, 257)
+MANY = tuple(1 + (7 * i) % 40 for i in range(70))   # more rows than one wave has lanes
+
+
+def _np(t):
+    return t.detach()[0].transpose(0, 1).float().cpu().numpy()
+
+
+@pytest.mark.parametrize("lengths,hq,hk,scale", [
+    (EDGES, 6, 2, 128 ** -0.5),     # 64-token blocks
+    (EDGES, 56, 8, 128 ** -0.5),    # 128-token blocks, 7:1 GQA
+    (EDGES, 52, 52, 128 ** -0.5),   # 128-token blocks, dK / dV written directly
+    (MANY, 4, 2, 128 ** -0.5),      # positions from the grid, 64-token blocks
+    (MANY, 60, 10, 128 ** -0.5),    # positions from the grid, 128-token blocks
+    ((40, 300), 4, 2, -0.07),
+    ((40, 300), 4, 2, 0.0),
+])
+def test_block_edges(device, lengths, hq, hk, scale):
+    t = sum(lengths)
+    print(f"case rows={len(lengths)} T={t} hq={hq} hk={hk} scale={scale}", flush=True)
+    gen = torch.Generator().manual_seed(t + hq)
+
+    def heads(h):
+        x = torch.randn((1, t, h * 128), generator=gen).half().to(device)
+        return x.view(1, t, h, 128).transpose(1, 2).requires_grad_()
+
+    q, k, v = heads(hq), heads(hk), heads(hk)
+    o = packed_causal_attention(q, k, v, lengths, scale)
+    assert torch.equal(o, packed_causal_attention(q, k, v, lengths, scale))
+    ref, _ = oattn.forward(_np(q), _np(k), _np(v), lengths, scale)
+    got = o.detach()[0].float().cpu().numpy().astype(np.float64)
+    np.testing.assert_allclose(got, ref, rtol=2e-3, atol=2e-3)
+    g = torch.randn((1, t, hq, 128), generator=gen).half().to(device)
+    grads = torch.autograd.grad(o, (q, k, v), g)
+    refs = oattn.backward(_np(q), _np(k), _np(v), g[0].float().cpu().numpy(), lengths, scale)
+    for name, x, ref_g in zip("qkv", grads, refs):
+        norm = np.linalg.norm(ref_g)
+        err = np.linalg.norm(_np(x).astype(np.float64) - ref_g)
+        assert err <= 1e-2 * norm, f"d{name}: {err:.3e} of {norm:.3e}"
