@@ -92,7 +92,6 @@ struct GemmParams {
   // term fp16(fp16(lz . lb^T) * lscale) here ([M][N]), which the reduce adds
   // instead of recomputing it from lora_B rows.
   half_t* lora_plane;
-  int pingpong;     // 8-wave NT configurations: ping-pong main loop (set by gemm_nt)
   // Dense NT kernels: A (B) stored K-major, element (m, k) at A[k * lda + m]
   // ((n, k) at B[k * ldb + n]), as a transposed view stores it; plain and
   // split-K epilogues only.
@@ -278,14 +277,14 @@ int gemm_nt(const GemmParams& p, int ct, int epi, hipStream_t stream, void* part
 bool staged_epilogue_enabled();
 // Split-K scratch that gemm_nt uses for an M x N x K product (0: no split):
 // the fp32 partial planes and an fp16 plane for a LoRA forward's rank term.
-size_t nt_partial_bytes(int64_t m, int64_t n, int64_t k);
-// Tile configuration (1..10 in gemm_nt.hip's list) and split-K plan of an
-// M x N x K product on the NT kernels.
+size_t nt_partial_bytes(int64_t m, int64_t n, int64_t k, int layout = 0);
+// Tile configuration (1..8 in gemm_nt.hip's list) and split-K plan of an
+// M x N x K product on the NT kernels (layout: bit 0 / 1 for K-major A / B).
 struct NtPlan {
   int cfg;
   int64_t splits, k_split;
 };
-NtPlan nt_plan(int64_t m, int64_t n, int64_t k);
+NtPlan nt_plan(int64_t m, int64_t n, int64_t k, int layout = 0);
 
 // Fused NF4 forward (gemm_nf4.hip): Y = X . Wdec^T with p.M = T, p.N = N,
 // p.K = K, p.A = X, p.w = the NF4 weight, the NT kernel's tile plan and

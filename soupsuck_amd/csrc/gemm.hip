@@ -1256,10 +1256,9 @@ extern "C" int ss_gemm_f16(int a_trans, int b_trans, int64_t m, int64_t n, int64
 
 extern "C" size_t ss_gemm_f16_workspace_size(int a_trans, int b_trans, int64_t m, int64_t n,
                                              int64_t k) {
-  // Split-K partials of the dense NT kernel (every operand layout).
-  (void)a_trans;
-  (void)b_trans;
-  return ss::nt_partial_bytes(m, n, k);
+  // Split-K partials of the dense NT kernel (a K-major A is a_trans, a K-major B is
+  // an untransposed b).
+  return ss::nt_partial_bytes(m, n, k, (a_trans ? 1 : 0) | (b_trans ? 0 : 2));
 }
 
 extern "C" int ss_gemm_f16_split(int a_trans, int b_trans, int64_t m, int64_t n, int64_t k,

@@ -532,8 +532,7 @@ __global__ __launch_bounds__(C::kThreads, C::MINW) void gemm_nf4_kernel(GemmPara
   nt_epilogue<C, CT, EPI>(p, m0, n0, acc, smem, split);
 }
 
-// Configurations (same tiles, waves and stage depth as the dense kernel's
-// configurations 1, 2 and 8).
+// Configurations (1, 2 and 8 in nf4_plan).
 using Nf4Small = NtCfg<64, 64, 2, 2, 32, 4, 2>;
 using Nf4Mid = NtCfg<128, 128, 2, 2, 32, 4, 2>;
 using Nf4Big = NtCfg<256, 256, 2, 4, 32, 4, 2>;
@@ -569,16 +568,45 @@ int dispatch_nf4t(const GemmParams& p, int64_t splits, hipStream_t stream) {
 
 }  // namespace
 
-// Tile plan of the fused kernel: the NT kernel's plan (configurations 1, 2
-// and 8 only), except for one or two 128-row tiles, where streaming the
+// Tile plan of the fused kernel.  One or two 128-row tiles, where streaming the
 // weight sets the pace: 64x64 tiles up to 64 rows, 128x128 above, split over
-// k until about 512 workgroups run, each split at least 512 deep.
-NtPlan nf4_plan(int64_t m, int64_t n, int64_t k) {
-  if (m > 256) {
-    NtPlan plan = nt_plan(m, n, k);
-    if (plan.cfg != 1 && plan.cfg != 2 && plan.cfg != 8) plan.cfg = 2;
-    return plan;
+// k until about 512 workgroups run, each split at least 512 deep.  More rows (only
+// without the decode-first path's scratch): 256x256 tiles once half the CUs get one,
+// 128x128 split over a long K, 64x64 split for a few tiles.
+static NtPlan nf4_wide_plan(int64_t m, int64_t n, int64_t k) {
+  NtPlan plan{1, 1, k};
+  const int64_t t256 = cdiv(m, 256) * cdiv(n, 256);
+  const int64_t t128 = cdiv(m, 128) * cdiv(n, 128);
+  int64_t s = 1;
+  if (t256 >= 96 && cdiv(m, 128) * cdiv(n, 256) <= 256 && k < 8192) {
+    plan.cfg = 2;
+  } else if (t256 >= 128) {
+    plan.cfg = 8;
+  } else if (k >= 32768) {
+    plan.cfg = 8;
+    s = 256 / t256 < k / 2048 ? 256 / t256 : k / 2048;
+  } else if (k >= 2048 && t128 < 256) {
+    plan.cfg = 2;
+    s = 512 / t128 < k / 1024 ? 512 / t128 : k / 1024;
+    if (s > 8) s = 8;
+  } else if (t256 >= 96) {
+    plan.cfg = 8;
+    s = 2;
+  } else if (t128 >= 128) {
+    plan.cfg = 2;
+  } else if (t128 < 64 && k >= 1024) {
+    s = 256 / (cdiv(m, 64) * cdiv(n, 64));
+    if (s > k / 384) s = k / 384;
+    if (s > 8) s = 8;
   }
+  if (s < 1) s = 1;
+  plan.k_split = cdiv(cdiv(k, s), 64) * 64;
+  plan.splits = cdiv(k, plan.k_split);
+  return plan;
+}
+
+NtPlan nf4_plan(int64_t m, int64_t n, int64_t k) {
+  if (m > 256) return nf4_wide_plan(m, n, k);
   NtPlan plan{m <= 64 ? 1 : 2, 1, k};
   const int64_t bm = plan.cfg == 1 ? 64 : 128;
   const int64_t tiles = cdiv(m, bm) * cdiv(n, bm);

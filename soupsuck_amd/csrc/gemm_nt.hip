@@ -7,13 +7,10 @@
 //
 // Operand layouts, configurations and the epilogue: nt_core.h.
 //
-// Per stage a wave runs BK / 16 MFMA k-steps; fragments are double buffered
-// so the reads of k-step kk+1 overlap the MFMAs of kk.  One s_barrier per
-// stage sits before the last k-step: by then every wave has read all its
-// fragments of stage kt (lgkmcnt(0)), so buffer kt % STAGES is refilled with
-// stage kt + STAGES right after it, and stage kt+1 (waited for with vmcnt
-// before the barrier) is read while the last MFMAs of stage kt run; the
-// refill DMAs are interleaved between those MFMAs.
+// Two main loops: NtStream (4 waves, 64-deep stages; every configuration that nt_plan
+// weighs) and the ping-pong loop of eight waves with 32-deep stages, which stays ahead
+// where A lies K-major (the cross-entropy's dW, 151936 x 1536 x 576: 320 us against 336
+// us on 128x128 stream tiles).
 //
 // The DMA is issued from inline asm.  The compiler does not know which LDS
 // buffer an outstanding LDS DMA writes, and would wait for all of them
@@ -21,17 +18,12 @@
 // explicit instead.
 
 #include "tuning.h"
-#include <stdlib.h>
 
 #include "nt_core.h"
 
 namespace ss {
 namespace {
 
-// acc += A[m0.., kbeg .. kbeg+klen) . B[n0.., same k]^T for one output tile:
-// the pipelined direct-to-LDS main loop.  All of the workgroup's LDS DMAs
-// have completed when it returns; the caller puts a barrier between two calls
-// (the last k-step's LDS reads of one call and the first DMAs of the next).
 // Operand sources of one workgroup's tile (both main loops): per-lane DMA
 // sources as 32-bit byte offsets from the per-stage operand base, and the
 // per-stage advance of that base.  Rows past M / N (row-major operands) or
@@ -127,104 +119,6 @@ struct NtFrags {
   }
 };
 
-template <class C, int L = 0>
-__device__ __forceinline__ void nt_mainloop(const GemmParams& p, int64_t m0, int64_t n0,
-                                            int64_t kbeg, int64_t klen, unsigned char* smem,
-                                            NtAcc<C>& acc) {
-  const int tid = threadIdx.x;
-  const int lane = tid & (kWave - 1);
-  const int wave = tid / kWave;
-  const int wm = wave / C::kWavesN;
-  const int wn = wave % C::kWavesN;
-  const uint32_t lds0 = lds_address(smem);
-  const NtSources<C, L> src(p, m0, n0, kbeg, wave, lane);
-  const uint32_t lds_a = __builtin_amdgcn_readfirstlane(lds0 + wave * C::kDmaA * 1024);
-  const uint32_t lds_b = __builtin_amdgcn_readfirstlane(lds0 + C::kTileA + wave * C::kDmaB * 1024);
-  const NtFrags<C, L> frags(lane, wm, wn);
-
-  auto dma_one = [&](int64_t kt, int stage, int idx) {
-    if (idx < C::kDmaA) {
-      dma16(src.a_off[idx], src.a_base + kt * src.a_step,
-            lds_a + stage * C::kStageBytes + idx * 1024);
-    } else {
-      const int j = idx - C::kDmaA;
-      dma16(src.b_off[j], src.b_base + kt * src.b_step, lds_b + stage * C::kStageBytes + j * 1024);
-    }
-  };
-  auto read_frags = [&](int64_t kt, int kk, half8 (&af)[C::FM], half8 (&bf)[C::FN]) {
-    const unsigned char* base = smem + (kt % C::STAGES) * C::kStageBytes;
-#pragma unroll
-    for (int i = 0; i < C::FM; ++i) af[i] = frags.a(base, kk, i);
-#pragma unroll
-    for (int j = 0; j < C::FN; ++j) bf[j] = frags.b(base, kk, j);
-  };
-  // MFMA phases raise the wave's issue priority (s_setprio 1), so a SIMD's
-  // other wave, in its load / LDS phase, does not delay them (measured +7 % at
-  // 8192^3, neutral at the layer shapes).
-  auto mfma_block = [&](const half8 (&af)[C::FM], const half8 (&bf)[C::FN]) {
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int i = 0; i < C::FM; ++i)
-#pragma unroll
-      for (int j = 0; j < C::FN; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bf[j], acc[i][j], 0, 0, 0);
-    __builtin_amdgcn_s_setprio(0);
-  };
-
-  constexpr int kS = C::STAGES;
-  constexpr int kMfma = C::FM * C::FN;
-  const int64_t ktiles = klen / C::BK;
-  half8 fa[2][C::FM], fb[2][C::FN];
-#pragma unroll
-  for (int s = 0; s < kS; ++s)
-    if (s < ktiles)
-#pragma unroll
-      for (int idx = 0; idx < C::kDma; ++idx) dma_one(s, s, idx);
-  if (ktiles > 0) {
-    wait_stages<C::kDma, kS - 1>((ktiles < kS ? ktiles : kS) - 1);
-    asm volatile("s_barrier" ::: "memory");
-    read_frags(0, 0, fa[0], fb[0]);
-  }
-  for (int64_t kt = 0; kt < ktiles; ++kt) {
-#pragma unroll
-    for (int kk = 0; kk + 1 < C::KK; ++kk) {
-      read_frags(kt, kk + 1, fa[(kk + 1) & 1], fb[(kk + 1) & 1]);
-      mfma_block(fa[kk & 1], fb[kk & 1]);
-    }
-    constexpr int kLast = (C::KK - 1) & 1;
-    const bool more = kt + 1 < ktiles;
-    const bool refill = kt + kS < ktiles;
-    if (more) {
-      // Stages requested so far: 0 .. min(kt + kS - 1, ktiles - 1); stage kt+1
-      // must have landed.  lgkmcnt(0): this wave's reads of stage kt are done,
-      // so buffer kt % kS may be refilled once every wave passed the barrier.
-      const int64_t last = kt + kS - 1 < ktiles - 1 ? kt + kS - 1 : ktiles - 1;
-      wait_stages<C::kDma, kS - 2>(last - (kt + 1));
-      __builtin_amdgcn_s_waitcnt(0xC07F);
-      asm volatile("s_barrier" ::: "memory");
-    }
-    const int refill_stage = (int)(kt % kS);
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int idx = 0; idx < kMfma; ++idx) {
-      if (idx == kMfma / 2 && more) read_frags(kt + 1, 0, fa[0], fb[0]);
-      acc[idx / C::FN][idx % C::FN] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-          fa[kLast][idx / C::FN], fb[kLast][idx % C::FN], acc[idx / C::FN][idx % C::FN], 0, 0,
-          0);
-      if (refill) {
-#pragma unroll
-        for (int d = idx * C::kDma / kMfma; d < (idx + 1) * C::kDma / kMfma; ++d)
-          dma_one(kt + kS, refill_stage, d);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    __builtin_amdgcn_s_setprio(0);
-#pragma unroll
-    for (int d = kMfma < C::kDma ? kMfma * (C::kDma / kMfma) : C::kDma; d < C::kDma; ++d)
-      if (refill) dma_one(kt + kS, refill_stage, d);
-  }
-}
-
 // Ping-pong main loop of the 8-wave configurations (two waves per SIMD:
 // wave w and w + 4).  Run in lockstep, the two waves of a SIMD issue their
 // MFMAs, LDS reads and barrier waits at the same time, and the MFMA pipe
@@ -239,8 +133,7 @@ __device__ __forceinline__ void nt_mainloop(const GemmParams& p, int64_t m0, int
 // and by waves 4-7 in phase 2kt + 1, and refilled (stage kt + STAGES) in read
 // phases from 2kt + 2 on; each wave's wait for its DMAs of stage kt + 1
 // precedes a barrier that ends before either group reads that stage.  The
-// MFMAs of every accumulator run in the order of nt_mainloop, so the results
-// are the same bit for bit.
+// MFMAs of every accumulator run in k order, as in NtStream: the same bits.
 template <class C, int L = 0>
 __device__ __forceinline__ void nt_mainloop_pp(const GemmParams& p, int64_t m0, int64_t n0,
                                                int64_t kbeg, int64_t klen, unsigned char* smem,
@@ -316,6 +209,142 @@ __device__ __forceinline__ void nt_mainloop_pp(const GemmParams& p, int64_t m0, 
   if (!late) barrier();
 }
 
+// Main loop of the 4-wave configurations with 64-deep stages (BK = 64): the DMAs fetch
+// 128-byte row pieces (64-byte pieces, as the 32-deep stages have, reach 25 B/clk/CU into
+// LDS; 256x128 tiles need 48), and the loop overlaps within a wave, not between waves:
+// every memory instruction has a slot between two MFMAs, spread evenly (bursts stall:
+// 16384 x 18944 x 3584 in 1771 us against 1803 us with the eight DMAs of a half stage
+// back to back, 1840 us with fourteen).  Per stage kt of four k-steps,
+//   k-steps 0 .. 2: the fragments of the next k-step;
+//   k-step 3: after kB MFMAs the wait for stage kt + 1 and the barrier, then the
+//   fragments of its k-step 0.
+// Stage kt's buffer was last read in k-step 2 (fragments of k-step 3), before the
+// barrier of k-step 3; the DMAs of stage kt + STAGES into it start after that barrier
+// and end before the next one.  Every accumulator adds its products in k order.
+template <class C, int L>
+struct NtStream {
+  static constexpr int kS = C::STAGES, kMf = C::FM * C::FN, kFr = C::FM + C::FN;
+  static constexpr int kB = kMf >= 8 ? 2 : kMf >= 2 ? 1 : 0;  // MFMAs of the last k-step before its barrier
+  static constexpr int kPart = kMf - kB;       // slots after it, in that k-step
+  // DMA d of a stage goes to slot at(d), counted from the barrier: spread over about
+  // half a stage when the next barrier waits for it (two buffers), else a whole one.
+  static constexpr int kSpan = kS == 2 ? 2 * kMf : 4 * kMf - (kMf >= 2 ? 2 : 0);
+  static constexpr int at(int d) { return (2 * d + 1) * kSpan / (2 * C::kDma); }
+  static constexpr int first_of(int slot) {  // DMAs before this slot
+    int n = 0;
+    while (n < C::kDma && at(n) < slot) ++n;
+    return n;
+  }
+  static constexpr int kEarly = first_of(kPart);  // DMAs issued within the barrier's k-step
+  static_assert(C::KK == 4 && (kS == 2 || kS == 3) && kSpan <= 4 * kMf, "stages");
+  const NtSources<C, L> src;
+  const NtFrags<C, L> frags;
+  const unsigned char* smem;
+  uint32_t lds_a, lds_b;
+
+  __device__ __forceinline__ NtStream(const GemmParams& p, int64_t m0, int64_t n0, int64_t kbeg,
+                                      unsigned char* lds, int wave, int lane)
+      : src(p, m0, n0, kbeg, wave, lane),
+        frags(lane, wave / C::kWavesN, wave % C::kWavesN),
+        smem(lds) {
+    const uint32_t lds0 = lds_address(lds);
+    lds_a = __builtin_amdgcn_readfirstlane(lds0 + wave * C::kDmaA * 1024);
+    lds_b = __builtin_amdgcn_readfirstlane(lds0 + C::kTileA + wave * C::kDmaB * 1024);
+  }
+  // buf: the stage's buffer.
+  __device__ __forceinline__ void dma(int64_t kt, int buf, int idx) const {
+    if (idx < C::kDmaA)
+      dma16(src.a_off[idx], src.a_base + kt * src.a_step, lds_a + buf * C::kStageBytes + idx * 1024);
+    else
+      dma16(src.b_off[idx - C::kDmaA], src.b_base + kt * src.b_step,
+            lds_b + buf * C::kStageBytes + (idx - C::kDmaA) * 1024);
+  }
+  __device__ __forceinline__ half8 frag(int buf, int kk, int f) const {
+    const unsigned char* base = smem + buf * C::kStageBytes;
+    return f < C::FN ? frags.b(base, kk, f) : frags.a(base, kk, f - C::FN);
+  }
+  static __device__ __forceinline__ int next_buf(int buf) { return buf + 1 == kS ? 0 : buf + 1; }
+  // Fragment read r of a k-step, in the order the MFMAs need them (B fragments and the
+  // first A fragment for the first row of blocks, then a row's A fragment each).
+  static constexpr int order(int r) { return r == 0 ? 0 : r == 1 ? C::FN : r <= C::FN ? r - 1 : r; }
+
+  // AHEAD: stages in flight beyond kt + 1 at its wait; REFILL / CONT: stage kt + kS (its
+  // first DMAs) / kt + kS - 1 (its other ones) exists; MORE: stage kt + 1 does.
+  template <int AHEAD, bool REFILL, bool CONT, bool MORE>
+  __device__ __forceinline__ void stage(int64_t kt, int buf, half8 (&f)[2][kFr],
+                                        NtAcc<C>& acc) const {
+    const int after = next_buf(buf);
+    const int before = buf == 0 ? kS - 1 : buf - 1;  // buffer of stages kt - 1 and kt + kS - 1
+#pragma unroll
+    for (int kk = 0; kk < C::KK; ++kk) {
+#pragma unroll
+      for (int s = 0; s < kMf; ++s) {
+        half8(&now)[kFr] = f[kk & 1];
+        half8(&next)[kFr] = f[(kk + 1) & 1];
+        const bool last = kk == C::KK - 1;
+        if (MORE && last && s == kB) {
+          wait_vm<AHEAD * C::kDma>();
+          __builtin_amdgcn_s_waitcnt(0xC07F);
+          asm volatile("s_barrier" ::: "memory");
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int r = 0; r < kFr; ++r) {
+          if (!last && s == r * kMf / kFr) next[order(r)] = frag(buf, kk + 1, order(r));
+          if (MORE && last && s == kB + r * kPart / kFr) next[order(r)] = frag(after, 0, order(r));
+        }
+        const int slot = last ? s - kB : kPart + kk * kMf + s;  // from the barrier
+#pragma unroll
+        for (int d = 0; d < C::kDma; ++d) {
+          if (at(d) != slot) continue;
+          if (last && s >= kB) {
+            if (REFILL) dma(kt + kS, buf, d);
+          } else if (!last) {
+            if (CONT) dma(kt + kS - 1, before, d);
+          }
+        }
+        const int i = s / C::FN, j = s % C::FN;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(now[C::FN + i], now[j], acc[i][j], 0,
+                                                           0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  __device__ __forceinline__ void run(int64_t ktiles, NtAcc<C>& acc) const {
+    if (ktiles <= 0) return;
+#pragma unroll
+    for (int st = 0; st < kS - 1; ++st)
+      if (st < ktiles)
+#pragma unroll
+        for (int idx = 0; idx < C::kDma; ++idx) dma(st, st, idx);
+    if (ktiles >= kS) {
+#pragma unroll
+      for (int idx = 0; idx < kEarly; ++idx) dma(kS - 1, kS - 1, idx);
+      wait_vm<(kS - 2) * C::kDma + kEarly>();
+    } else {
+      wait_vm<0>();
+    }
+    asm volatile("s_barrier" ::: "memory");
+    half8 f[2][kFr];
+#pragma unroll
+    for (int i = 0; i < kFr; ++i) f[0][order(i)] = frag(0, 0, order(i));
+    __builtin_amdgcn_sched_barrier(0);
+    int64_t kt = 0;
+    int buf = 0;
+    for (; kt < ktiles - kS; ++kt, buf = next_buf(buf))
+      stage<kS - 2, true, true, true>(kt, buf, f, acc);
+    if (kt == ktiles - kS) {
+      stage<kS - 2, false, true, true>(kt++, buf, f, acc);
+      buf = next_buf(buf);
+    }
+    if (kS == 3 && kt == ktiles - 2) {
+      stage<0, false, false, true>(kt++, buf, f, acc);
+      buf = next_buf(buf);
+    }
+    stage<0, false, false, false>(kt, buf, f, acc);
+  }
+};
+
 // LDS of a GEMM workgroup: the stage ring; for the dX epilogue (rank-16
 // update) also room for a rank-16 grad tail block.
 template <class C, int EPI>
@@ -357,13 +386,12 @@ __global__ __launch_bounds__(C::kThreads, C::MINW) void gemm_nt_kernel(GemmParam
   for (int i = 0; i < C::FM; ++i)
 #pragma unroll
     for (int j = 0; j < C::FN; ++j) acc[i][j] = float16v{};
-  if constexpr (C::kWaves == 8 && C::KK == 2) {
-    if (p.pingpong)
-      nt_mainloop_pp<C, L>(p, m0, n0, kbeg, klen, smem, acc);
-    else
-      nt_mainloop<C, L>(p, m0, n0, kbeg, klen, smem, acc);
+  if constexpr (C::kWaves == 4 && C::BK == 64) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    NtStream<C, L>(p, m0, n0, kbeg, smem, wave, threadIdx.x & (kWave - 1))
+        .run(klen / C::BK, acc);
   } else {
-    nt_mainloop<C, L>(p, m0, n0, kbeg, klen, smem, acc);
+    nt_mainloop_pp<C, L>(p, m0, n0, kbeg, klen, smem, acc);
   }
   static_assert(!GluStage<C>::kOk || GluStage<C>::kBytes <= nt_smem_bytes<C, EPI>(), "stage");
   nt_epilogue<C, CT, EPI>(p, m0, n0, acc, smem, split);
@@ -522,17 +550,21 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmParams p, int sp
   }
 }
 
+// The rank-16 grad tails on their own.
+__global__ __launch_bounds__(256) void rank_tail_kernel(GemmParams p) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[kRankGradSmem];
+  run_tail_block(p, blockIdx.x, smem);
+}
+
 // Tile configurations: <BM, BN, waves M, waves N, BK, stages, min waves/SIMD>.
-using NtSmall = NtCfg<64, 64, 2, 2, 32, 4, 2>;      // 4 waves of 32x32, 32 KiB LDS
-using NtMid = NtCfg<128, 128, 2, 2, 32, 3, 2>;      // 4 waves of 64x64, 48 KiB LDS
-using NtBig4 = NtCfg<256, 256, 2, 2, 32, 3, 1>;     // 4 waves of 128x128, 96 KiB LDS
-using NtBig8 = NtCfg<256, 256, 2, 4, 64, 2, 2>;     // 8 waves of 128x64, 128 KiB LDS
-using NtWide8 = NtCfg<256, 128, 4, 2, 64, 2, 2>;    // 8 waves of 64x64, 96 KiB LDS
-using NtBig8s = NtCfg<256, 256, 2, 4, 32, 3, 2>;    // 8 waves of 128x64, 96 KiB LDS
-using NtMid64 = NtCfg<128, 128, 2, 2, 64, 2, 2>;    // 4 waves of 64x64, 64 KiB LDS
-using NtBig8s4 = NtCfg<256, 256, 2, 4, 32, 4, 2>;   // 8 waves of 128x64, 128 KiB LDS
-using NtWide8s4 = NtCfg<256, 128, 4, 2, 32, 4, 1>;  // 8 waves of 64x64, 96 KiB LDS
-using NtTall8s4 = NtCfg<128, 256, 2, 4, 32, 4, 1>;  // 8 waves of 64x64, 96 KiB LDS
+using Nt64 = NtCfg<64, 64, 2, 2, 64, 3, 2>;         // 1: 4 waves of 32x32, 48 KiB LDS
+using Nt128x64 = NtCfg<128, 64, 2, 2, 64, 3, 2>;    // 2: 64x32, 72 KiB
+using Nt128 = NtCfg<128, 128, 2, 2, 64, 3, 1>;      // 3: 64x64, 96 KiB
+using Nt128x256 = NtCfg<128, 256, 2, 2, 64, 3, 1>;  // 4: 64x128, 144 KiB
+using Nt256x160 = NtCfg<256, 160, 4, 1, 64, 3, 1>;  // 5: 64x160, 156 KiB
+using Nt256x192 = NtCfg<256, 192, 2, 2, 64, 2, 1>;  // 6: 128x96, 112 KiB
+using Nt256 = NtCfg<256, 256, 2, 2, 64, 2, 1>;      // 7: 128x128, 128 KiB
+using NtPingPong = NtCfg<256, 256, 2, 4, 32, 4, 2>; // 8: 8 waves of 128x64, 128 KiB
 
 template <class C, int CT, int EPI, int L = 0>
 int launch_nt(const GemmParams& p, int64_t splits, hipStream_t stream) {
@@ -545,17 +577,14 @@ int launch_nt(const GemmParams& p, int64_t splits, hipStream_t stream) {
   return SS_OK;
 }
 
-// K-major operands (L != 0) take the configurations nt_plan picks (1, 2, 8, 9,
-// 10); the others are reached only through a build-time override and keep
-// row-major operands.
+// K-major operands (L != 0): configurations 1, 3, 4 and 8 (nt_plan's mask).
 template <int CT, int EPI, int L>
 int dispatch_nt_t(const GemmParams& p, int cfg, int64_t splits, hipStream_t stream) {
   switch (cfg) {
-    case 10: return launch_nt<NtTall8s4, CT, EPI, L>(p, splits, stream);
-    case 9: return launch_nt<NtWide8s4, CT, EPI, L>(p, splits, stream);
-    case 8: return launch_nt<NtBig8s4, CT, EPI, L>(p, splits, stream);
-    case 2: return launch_nt<NtMid, CT, EPI, L>(p, splits, stream);
-    case 1: return launch_nt<NtSmall, CT, EPI, L>(p, splits, stream);
+    case 1: return launch_nt<Nt64, CT, EPI, L>(p, splits, stream);
+    case 3: return launch_nt<Nt128, CT, EPI, L>(p, splits, stream);
+    case 4: return launch_nt<Nt128x256, CT, EPI, L>(p, splits, stream);
+    case 8: return launch_nt<NtPingPong, CT, EPI, L>(p, splits, stream);
     default: return SS_ERR_UNSUPPORTED;
   }
 }
@@ -571,16 +600,14 @@ int dispatch_nt(const GemmParams& p, int cfg, int64_t splits, hipStream_t stream
     if (layout) return SS_ERR_UNSUPPORTED;
   }
   switch (cfg) {
-    case 10: return launch_nt<NtTall8s4, CT, EPI>(p, splits, stream);
-    case 9: return launch_nt<NtWide8s4, CT, EPI>(p, splits, stream);
-    case 8: return launch_nt<NtBig8s4, CT, EPI>(p, splits, stream);
-    case 7: return launch_nt<NtMid64, CT, EPI>(p, splits, stream);
-    case 6: return launch_nt<NtBig8s, CT, EPI>(p, splits, stream);
-    case 5: return launch_nt<NtWide8, CT, EPI>(p, splits, stream);
-    case 4: return launch_nt<NtBig8, CT, EPI>(p, splits, stream);
-    case 3: return launch_nt<NtBig4, CT, EPI>(p, splits, stream);
-    case 2: return launch_nt<NtMid, CT, EPI>(p, splits, stream);
-    default: return launch_nt<NtSmall, CT, EPI>(p, splits, stream);
+    case 1: return launch_nt<Nt64, CT, EPI>(p, splits, stream);
+    case 2: return launch_nt<Nt128x64, CT, EPI>(p, splits, stream);
+    case 3: return launch_nt<Nt128, CT, EPI>(p, splits, stream);
+    case 4: return launch_nt<Nt128x256, CT, EPI>(p, splits, stream);
+    case 5: return launch_nt<Nt256x160, CT, EPI>(p, splits, stream);
+    case 6: return launch_nt<Nt256x192, CT, EPI>(p, splits, stream);
+    case 7: return launch_nt<Nt256, CT, EPI>(p, splits, stream);
+    default: return SS_ERR_UNSUPPORTED;
   }
 }
 
@@ -599,80 +626,61 @@ bool aligned16(const void* ptr) { return reinterpret_cast<uintptr_t>(ptr) % 16 =
 
 }  // namespace
 
-// Configuration and split-K plan for an M x N x K product.
-//   128x256 (8 waves) when 96 or more 256x256 tiles would run but the
-//   128x256 tiles still fit one wave on the CUs (K < 8192);
-//   256x256 (8 waves, 4-stage ring) once it gives at least half the CUs a
-//   tile;
-//   a very long K (32768 or more) over at most 128 tiles of 256x256: those
-//   tiles split over k into one wave of workgroups;
-//   long K with few 128x128 tiles: split over k (each split at least 1024
-//   k), 256x128 tiles with about one workgroup per CU where M fills 256-row
-//   tiles, else 128x128 with about 512 workgroups;
-//   96..127 tiles of 256x256 and a long K: 256x256 split in two;
-//   128x128 while it gives half the CUs a tile; else 64x64.
-// SS_TUNE_NT_TILE (1..10, the cases of dispatch_nt) and
-// SS_TUNE_NT_SPLITS override the choice (build-time constants, tuning.h).
-NtPlan nt_plan(int64_t m, int64_t n, int64_t k) {
-  constexpr int forced = SS_TUNE_NT_TILE;
-  constexpr int forced_splits = SS_TUNE_NT_SPLITS;
+// Configuration and split-K plan for an M x N x K product: the cheapest by a cost model
+// of the time a launch takes,
+//   start + q (tile + stages (stage + load f)),   q = ceil(workgroups / CUs),
+// with a configuration's start, epilogue and 64-deep stage times in us and f the busy
+// share of the CUs (with all of them busy the clock falls), plus a split's reduce.
+// The constants are least-squares fits to 156 products of this kernel measured on
+// MI355X (M 260 .. 16384 at the Qwen2.5 1.5B and 7B projection shapes, every
+// configuration and up to 5 splits); the model's choice takes 1.02 times the best
+// measured one on average, 1.10 at the 95th percentile.  Against the former rules and
+// kernels (32-deep stages, tiles by thresholds on the tile count), us before -> after:
+// 990 x 1536 x 1536 16.5 -> 9.7, 990 x 256 x 1536 11.9 -> 6.7, 990 x 8960 x 1536 35.4 ->
+// 29.2, 826 x 8960 x 1536 32.9 -> 25.7, 990 x 1536 x 8960 43.7 -> 38.5, 990 x 3584 x 3584
+// 44.2 -> 29.5, 2048 x 3584 x 3584 62.2 -> 50.3, 16384 x 18944 x 3584 1898 -> 1771.
+struct TileCost {
+  int cfg, bm, bn;
+  float start, tile, stage, load;
+};
+constexpr TileCost kTileCosts[] = {
+    {1, 64, 64, 3.6f, 0.0f, 0.151f, 0.043f},     {2, 128, 64, 3.8f, 0.0f, 0.227f, 0.094f},
+    {3, 128, 128, 1.6f, 2.6f, 0.281f, 0.196f},   {4, 128, 256, 0.0f, 6.4f, 0.460f, 0.322f},
+    {5, 256, 160, 0.0f, 7.7f, 0.553f, 0.393f},   {6, 256, 192, 0.0f, 7.6f, 0.711f, 0.468f},
+    {7, 256, 256, 0.0f, 13.1f, 0.896f, 0.532f},
+};
+
+// layout: bit 0 / 1 for K-major A / B (GemmParams::a_t, b_t).
+NtPlan nt_plan(int64_t m, int64_t n, int64_t k, int layout) {
+  const int64_t cus = device_cu_count();
   NtPlan plan{1, 1, k};
-  const int64_t t256 = cdiv(m, 256) * cdiv(n, 256);
-  const int64_t t128 = cdiv(m, 128) * cdiv(n, 128);
-  const int64_t t10 = cdiv(m, 128) * cdiv(n, 256);  // 128x256 tiles
-  if (t256 >= 96 && t10 <= 256 && k < 8192) {
-    // 96 or more tiles of 256x256, but one wave of 128x256 tiles (8 waves):
-    // the half-height tiles fill the CUs better and pad M less (2048 x 3584
-    // x 3584: 60.8 vs 67.3 us for 256x256, 70.6 us for 128x128; the
-    // cross-entropy chunk 826 x 8192 x 1536: 31.5 vs 37.7 us).
-    plan.cfg = 10;
-  } else if (t256 >= 128) {
+  if ((layout & 1) && cdiv(m, 256) * cdiv(n, 256) >= cus / 2) {
     plan.cfg = 8;
-  } else if (k >= 32768 && t256 <= 128) {
-    // A very long K over few output tiles (the cross-entropy dX over the whole
-    // vocabulary, 523 x 1536 x 151936): 256x256 tiles split over K into one wave
-    // of workgroups, one 8-wave workgroup per CU (14 splits: 403 us against 485
-    // us for 128x128 split 8; 16 or 18 splits, a second partial wave: 490 us).
-    plan.cfg = 8;
-    int64_t s = 256 / t256;
-    if (s > k / 2048) s = k / 2048;
-    plan.splits = s < 1 ? 1 : s;
-  } else if (k >= 2048 && t128 < 256) {
-    plan.cfg = 2;
-    int64_t s = 512 / t128;
-    if (s > k / 1024) s = k / 1024;
-    plan.splits = s < 1 ? 1 : (s > 8 ? 8 : s);
-    // 256x128 tiles (8 waves) when M fills 256-row tiles as well as 128-row
-    // ones and a split of about one workgroup per CU still gives 192 or more
-    // workgroups (990 x 1536 x 8960: 44 us against 50 us for 128x128).
-    const int64_t tw = cdiv(m, 256) * cdiv(n, 128);
-    int64_t sw = 256 / tw;
-    if (sw > k / 1024) sw = k / 1024;
-    sw = sw < 1 ? 1 : (sw > 8 ? 8 : sw);
-    if (cdiv(m, 256) * 2 == cdiv(m, 128) && tw * sw >= 192) {
-      plan.cfg = 9;
-      plan.splits = sw;
-    }
-  } else if (t256 >= 96) {
-    // 96..127 tiles of 256x256 with a long K (k >= 8192 here): 256x256 split
-    // in two (2048 x 3584 x 18944: 263 vs 295 us for 128x256, 354 us for
-    // 128x128).
-    plan.cfg = 8;
-    plan.splits = 2;
-  } else if (t128 >= 128) {
-    plan.cfg = 2;
-  } else if (t128 < 64 && k >= 1024) {
-    // Few output tiles (e.g. a 256-wide k/v projection): 64x64 tiles split
-    // over K until about 256 workgroups run, each split at least 384 deep.
-    const int64_t t64 = cdiv(m, 64) * cdiv(n, 64);
-    int64_t s = 256 / t64;
-    if (s > k / 384) s = k / 384;
-    plan.splits = s < 1 ? 1 : (s > 8 ? 8 : s);
+    return plan;
   }
-  if (forced >= 1 && forced <= 10) plan.cfg = forced;
-  if (forced_splits >= 1) plan.splits = forced_splits;
-  plan.k_split = cdiv(cdiv(k, plan.splits), 64) * 64;
-  plan.splits = cdiv(k, plan.k_split);
+  // Splits: at least 512 deep; more than 8 only where each still has 8192.
+  int64_t most = k / 512 < 8 ? k / 512 : (k / 8192 > 8 ? k / 8192 : 8);
+  if (most > 16) most = 16;
+  if (most < 1) most = 1;
+  float best = 0.0f;
+  for (const TileCost& c : kTileCosts) {
+    if (layout && c.cfg != 1 && c.cfg != 3 && c.cfg != 4) continue;
+    const int64_t tiles = cdiv(m, c.bm) * cdiv(n, c.bn);
+    for (int64_t s = 1; s <= most; ++s) {
+      const int64_t k_split = cdiv(cdiv(k, s), 64) * 64;
+      if (cdiv(k, k_split) != s) continue;
+      const int64_t q = cdiv(tiles * s, cus);
+      const float f = (float)(tiles * s) / (float)(q * cus);
+      const float stages = (float)(k_split / 64);
+      float us = c.start + (float)q * (c.tile + stages * (c.stage + c.load * f));
+      if (s > 1) us += 5.4f + ((float)s * 1.01f + 0.29f) * (float)m * (float)n * 1e-6f;
+      if (best == 0.0f || us < best) {
+        best = us;
+        plan = NtPlan{c.cfg, s, k_split};
+      }
+    }
+  }
+  if (plan.splits == 1) plan.k_split = k;
   return plan;
 }
 
@@ -696,15 +704,11 @@ static size_t nt_split_bytes(int64_t m, int64_t n, int64_t splits) {
   return nt_plane_offset(m, n, splits) + (size_t)(m * n) * sizeof(half_t);
 }
 
-size_t nt_partial_bytes(int64_t m, int64_t n, int64_t k) {
+size_t nt_partial_bytes(int64_t m, int64_t n, int64_t k, int layout) {
   if (m <= 0 || n <= 0 || k <= 0 || k % 64 != 0) return 0;
-  const NtPlan plan = nt_plan(m, n, k);
+  const NtPlan plan = nt_plan(m, n, k, layout);
   return plan.splits > 1 ? nt_split_bytes(m, n, plan.splits) : 0;
 }
-
-// SS_TUNE_NT_PINGPONG = 0 keeps the 8-wave configurations on the lockstep
-// main loop (tuning.h).
-static bool pingpong_enabled() { return SS_TUNE_NT_PINGPONG != 0; }
 
 // SS_TUNE_NT_STAGED = 0 keeps fp16 epilogues on direct 2-byte stores.
 bool staged_epilogue_enabled() { return SS_TUNE_NT_STAGED != 0; }
@@ -712,7 +716,6 @@ bool staged_epilogue_enabled() { return SS_TUNE_NT_STAGED != 0; }
 int gemm_nt(const GemmParams& p0, int ct, int epi, hipStream_t stream, void* partials,
             size_t partial_bytes) {
   GemmParams p = p0;
-  p.pingpong = pingpong_enabled();
   p.c_vec = staged_epilogue_enabled() && ct == SS_F16 && !p.beta && p.N % 8 == 0 &&
             p.ldc % 8 == 0 && aligned16(p.C);
   if (p.M <= 0 || p.N <= 0 || p.K <= 0 || p.K % 64 != 0) return SS_ERR_UNSUPPORTED;  // K % 64
@@ -731,18 +734,19 @@ int gemm_nt(const GemmParams& p0, int ct, int epi, hipStream_t stream, void* par
   if (epi != EPI_PLAIN && (!aligned16(p.lz) || (epi == EPI_LORA && !aligned16(p.lb))))
     return SS_ERR_UNSUPPORTED;
   if (ct != SS_F16 && epi != EPI_PLAIN) return SS_ERR_UNSUPPORTED;
-  NtPlan plan = nt_plan(p.M, p.N, p.K);
+  NtPlan plan = nt_plan(p.M, p.N, p.K, (p.a_t ? 1 : 0) | (p.b_t ? 2 : 0));
   const size_t need = nt_split_bytes(p.M, p.N, plan.splits);
   if (plan.splits > 1 && (!partials || partial_bytes < need ||
                           reinterpret_cast<uintptr_t>(partials) % 16 != 0)) {
     plan.splits = 1;
     plan.k_split = p.K;
   }
-  // The rank-16 grad tail rides on unsplit dX products (rank-16 epilogue)
-  // after the GEMM tiles: measured, it fills idle CUs there (down / q / o / k
-  // / v backward 6-11 us faster).  On the split-K launches of the long-K dX it
-  // slowed the GEMM more than a launch of its own costs; there it leads the
-  // reduce launch instead.
+  // The rank-16 grad tail rides on unsplit dX products (rank-16 epilogue) after the GEMM
+  // tiles where the tile's LDS lets two or more workgroups share a CU (64 columns: it
+  // fills CUs that the GEMM leaves idle; q / o / k / v backward 6-11 us faster).  Behind
+  // the larger tiles, one workgroup per CU, it gets a launch of its own (990 x 8960 x 1536
+  // with 656 tail blocks: 50 us together, 34 + 7 us apart).  On the split-K launches of
+  // the long-K dX it slowed the GEMM more than a launch costs; there it leads the reduce.
   if (epi != EPI_RANK) p.tail_blocks = p.tail2_blocks = 0;
   if (p.tail_blocks + p.tail2_blocks > 0 && p.tail_ran) *p.tail_ran = 1;
   if (plan.splits > 1) {
@@ -779,7 +783,17 @@ int gemm_nt(const GemmParams& p0, int ct, int epi, hipStream_t stream, void* par
   }
   if (ct == SS_F16) {
     if (epi == EPI_LORA) return dispatch_nt<SS_F16, EPI_LORA>(p, plan.cfg, 1, stream);
-    if (epi == EPI_RANK) return dispatch_nt<SS_F16, EPI_RANK>(p, plan.cfg, 1, stream);
+    if (epi == EPI_RANK) {
+      const int64_t tails = p.tail_blocks + p.tail2_blocks;
+      if (tails == 0 || plan.cfg <= 2) return dispatch_nt<SS_F16, EPI_RANK>(p, plan.cfg, 1, stream);
+      GemmParams q = p;
+      q.tail_blocks = q.tail2_blocks = 0;
+      const int rc = dispatch_nt<SS_F16, EPI_RANK>(q, plan.cfg, 1, stream);
+      if (rc) return rc;
+      hipLaunchKernelGGL(rank_tail_kernel, dim3((unsigned)tails), dim3(256), 0, stream, p);
+      SS_CHECK_LAUNCH("rank_tail_kernel");
+      return SS_OK;
+    }
     if (p.glu) return dispatch_nt<SS_F16, EPI_GLU>(p, plan.cfg, 1, stream);
     return dispatch_nt<SS_F16, EPI_PLAIN>(p, plan.cfg, 1, stream);
   }

@@ -8,8 +8,8 @@
 // LDS (lane i at +16 i).  How many bytes of a row one DMA fetches sets the
 // DMA throughput (measured on MI355X, L2-resident data: 128 B per row ->
 // 43 B/clk/CU into LDS, 64 B -> 25, 32 B -> 14), so:
-//   BK = 64: a DMA covers 8 rows x 128 B.  Block b (rows 8b .. 8b+7) is 1 KiB;
-//     chunk c of row 8b + r sits at slot (c ^ (b & 1)) * 8 + r.
+//   BK = 64: a DMA covers 8 rows x 128 B, eight consecutive lanes on one row.
+//     Row r is 128 B; chunk c sits at chunk c ^ swz64(r), swz64(r) = (r >> 1) & 7.
 //   BK = 32: a DMA covers 16 rows x 64 B.  Row r is 64 B; chunk c sits at
 //     chunk c ^ swz32(r), swz32(r) = ((r >> 1) & 3) ^ ((r >> 3) & 1).
 // A 128-bit LDS read is served 16 lanes at a time over 64 four-byte banks
@@ -83,7 +83,8 @@ __device__ __forceinline__ void wait_stages(int64_t ahead) {
   wait_vm<0>();
 }
 
-// Chunk swizzle of the BK = 32 layout (see the layout notes above).
+// Chunk swizzles (see the layout notes above).
+__device__ __forceinline__ int swz64(int r) { return (r >> 1) & 7; }
 __device__ __forceinline__ int swz32(int r) { return ((r >> 1) & 3) ^ ((r >> 3) & 1); }
 
 // DMA g of an operand tile: the row and logical 16-byte chunk that lane
@@ -91,8 +92,8 @@ __device__ __forceinline__ int swz32(int r) { return ((r >> 1) & 3) ^ ((r >> 3) 
 template <int BK>
 __device__ __forceinline__ void dma_source(int g, int lane, int& row, int& chunk) {
   if constexpr (BK == 64) {
-    row = g * 8 + (lane & 7);
-    chunk = (lane >> 3) ^ (g & 1);
+    row = g * 8 + (lane >> 3);
+    chunk = (lane & 7) ^ swz64(row);
   } else {
     row = g * 16 + (lane >> 2);
     chunk = (lane & 3) ^ swz32(row);
@@ -107,8 +108,7 @@ __device__ __forceinline__ int frag_offset(int lane, int kk) {
   const int r = lane & 31;
   const int c = 2 * kk + (lane >> 5);
   if constexpr (BK == 64) {
-    const int b = r >> 3;
-    return b * 1024 + ((((c ^ (b & 1)) * 8) + (r & 7)) << 4);
+    return r * 128 + ((c ^ swz64(r)) << 4);
   } else {
     return r * 64 + ((c ^ swz32(r)) << 4);
   }
@@ -232,9 +232,9 @@ struct GluStage {
   static constexpr int kPitch = C::BN + 8;  // halves per staged row (bank spread)
   static constexpr int kChunksRow = C::BN / 8;
   static constexpr int kPer = C::WM * kChunksRow / C::kThreads;
-  static constexpr int kBatch = kPer < 4 ? kPer : 4;
+  static constexpr int kBatch = kPer <= 5 ? kPer : 4;
   static constexpr int kBytes = C::WM * kPitch * 2;
-  static constexpr bool kOk = C::WM * kChunksRow % C::kThreads == 0 && kPer >= 1 && kPer <= 8 &&
+  static constexpr bool kOk = C::WM * kChunksRow % C::kThreads == 0 && kPer >= 1 && kPer <= 16 &&
                               kPer % kBatch == 0;
 };
 
@@ -398,9 +398,14 @@ __device__ __forceinline__ void nt_epilogue_staged(const GemmParams& p, int64_t 
   load_bias<C>(p, n0, wn, lr, bias);
   wait_vm<0>();
   __syncthreads();
+  // One pass over the whole tile where the ring has room for it, else a pass per wave row
+  // group (whose waves then convert while the others wait).
+  constexpr int kGroups = C::BM / C::WM;
+  constexpr bool kWhole = kGroups * G::kBytes <= C::STAGES * C::kStageBytes;
+  constexpr int kPasses = kWhole ? 1 : kGroups;
 #pragma unroll 1
-  for (int q = 0; q < C::BM / C::WM; ++q) {
-    if (wm == q) {
+  for (int q = 0; q < kPasses; ++q) {
+    if (kWhole || wm == q) {
 #pragma unroll
       for (int i = 0; i < C::FM; ++i) {
 #pragma unroll
@@ -411,7 +416,7 @@ __device__ __forceinline__ void nt_epilogue_staged(const GemmParams& p, int64_t 
           const float b = bias[j];
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            const int row_l = i * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
+            const int row_l = (kWhole ? wm * C::WM : 0) + i * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
             half_t h;
             if constexpr (EPI == EPI_LORA) {
               const float y = (float)f32_to_f16(acc[i][j][r] * p.alpha + b);
@@ -430,7 +435,7 @@ __device__ __forceinline__ void nt_epilogue_staged(const GemmParams& p, int64_t 
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < G::kPer; ++k) {
+    for (int k = 0; k < G::kPer * (kWhole ? kGroups : 1); ++k) {
       const int c = tid + k * C::kThreads;
       const int row_l = c / G::kChunksRow;
       const int c8 = (c % G::kChunksRow) * 8;

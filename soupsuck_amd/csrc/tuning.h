@@ -36,17 +36,6 @@
 #ifndef SS_TUNE_NF4_DX_FUSED
 #define SS_TUNE_NF4_DX_FUSED 1
 #endif
-// NT kernel configuration (0 automatic, 1..10) and split count (0 automatic).
-#ifndef SS_TUNE_NT_TILE
-#define SS_TUNE_NT_TILE 0
-#endif
-#ifndef SS_TUNE_NT_SPLITS
-#define SS_TUNE_NT_SPLITS 0
-#endif
-// Ping-pong main loop of the 8-wave NT configurations (1 on, 0 lockstep).
-#ifndef SS_TUNE_NT_PINGPONG
-#define SS_TUNE_NT_PINGPONG 1
-#endif
 // fp16 epilogues staged through LDS with 16-byte row stores (1 on, 0 off).
 #ifndef SS_TUNE_NT_STAGED
 #define SS_TUNE_NT_STAGED 1
