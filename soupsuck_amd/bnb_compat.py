@@ -27,7 +27,7 @@ import torch
 
 from . import _lib
 from .kernels.nf4 import _validate_state, dequantize_nf4
-from .kernels.nf4_gemm import NF4Linear
+from .kernels.nf4_gemm import nf4_linear
 
 
 def dynamic_map_signed():
@@ -213,7 +213,7 @@ def matmul_4bit(A, B, quant_state, out=None, bias=None):
     if out is not None:
         raise NotImplementedError("out= is not supported")
     packed = B.t() if B.ndim == 2 and B.shape[0] == 1 else B
-    return NF4Linear.apply(A, packed, quant_state, bias)
+    return nf4_linear(A, packed, quant_state, bias)
 
 
 class Params4bit(torch.nn.Parameter):

@@ -138,9 +138,9 @@ def build_matmul(original, module):
     def matmul_4bit(A, B, quant_state, out=None, bias=None):
         packed = B.t() if isinstance(B, torch.Tensor) and B.ndim == 2 and B.shape[0] == 1 else B
         if enabled() and _matmul_route_ok(A, packed, quant_state, out, bias):
-            from .kernels.nf4_gemm import NF4Linear
+            from .kernels.nf4_gemm import nf4_linear
 
-            return NF4Linear.apply(A, packed, quant_state, bias)
+            return nf4_linear(A, packed, quant_state, bias)
         return original(A, B, quant_state, out=out, bias=bias)
 
     return matmul_4bit

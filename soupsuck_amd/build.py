@@ -1,6 +1,7 @@
 """Build the gfx950 shared library ``libsoupsuck_amd.so`` in-tree with hipcc.
 
-One hipcc invocation compiles every ``csrc/*.hip`` source for gfx950 only.
+One hipcc invocation compiles every ``csrc/*.hip`` source for gfx950 only; g++ then
+compiles the native autograd nodes (csrc/torch/nodes.cpp) against torch.
 Flags:
   -ffp-contract=off   keep a*b+c as two roundings (the reference launches every
                       kernel with enable_fp_fusion=False); bit-exact NF4 decode
@@ -18,6 +19,8 @@ from pathlib import Path
 PACKAGE = Path(__file__).resolve().parent
 CSRC = PACKAGE / "csrc"
 LIBRARY = PACKAGE / "libsoupsuck_amd.so"
+NODES = CSRC / "torch" / "nodes.cpp"    # autograd nodes over the C ABI (host code only)
+NATIVE = PACKAGE / "_native.so"
 ARCH = "gfx950"
 
 
@@ -30,6 +33,34 @@ def hipcc():
 
 def sources():
     return sorted(str(p) for p in CSRC.glob("*.hip"))
+
+
+def _nodes_command(target):
+    """g++ command of the native autograd nodes against this interpreter's torch."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+
+    command = ["g++", "-O2", "-fPIC", "-std=c++17", "-shared", "-D__HIP_PLATFORM_AMD__=1",
+               "-DUSE_ROCM=1", "-I", str(PACKAGE.parent / "include")]
+    for path in [*cpp_extension.include_paths(), "/opt/rocm/include",
+                 sysconfig.get_paths()["include"]]:
+        command += ["-isystem", path]
+    command += [str(NODES), "-o", str(target)]
+    for path in cpp_extension.library_paths():
+        command += ["-L" + path]
+    return command + ["-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip",
+                      "-L" + str(PACKAGE), "-l:" + LIBRARY.name, "-Wl,-rpath,$ORIGIN"]
+
+
+def build_nodes():
+    """Compile the native autograd nodes (links the kernel library, built before)."""
+    tmp = str(NATIVE) + ".tmp"
+    res = subprocess.run(_nodes_command(tmp), stdout=subprocess.PIPE, stderr=subprocess.STDOUT)
+    if res.returncode != 0:
+        raise RuntimeError("native nodes failed:\n" + res.stdout.decode(errors="replace"))
+    os.replace(tmp, NATIVE)
+    return NATIVE
 
 
 def build(verbose=False, jobs=None, address_sanitizer=False):
@@ -79,6 +110,8 @@ def build(verbose=False, jobs=None, address_sanitizer=False):
     if res.returncode != 0:
         raise RuntimeError("link failed:\n" + res.stdout.decode(errors="replace"))
     os.replace(tmp, target)
+    if not address_sanitizer:
+        build_nodes()
     return target
 
 
@@ -89,6 +122,9 @@ def built_library(address_sanitizer=False):
         list((PACKAGE.parent / "include").glob("*.h"))
     if not target.exists() or target.stat().st_mtime < max(p.stat().st_mtime for p in inputs):
         return build(address_sanitizer=address_sanitizer)
+    if not address_sanitizer and (not NATIVE.exists()
+                                  or NATIVE.stat().st_mtime < NODES.stat().st_mtime):
+        build_nodes()
     return target
 
 

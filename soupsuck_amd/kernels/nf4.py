@@ -94,8 +94,41 @@ FLAT_RULES = (
 )
 
 
+def _accepted(packed, state):
+    """The (N, K) shape of a state that keeps every rule of NESTED_STATE_RULES, in one pass
+    without the rules' namespace and calls, else None (the rules then name what is wrong)."""
+    try:
+        second, shape, offset = state.state2, state.shape, state.offset
+        n, k = shape
+        buffers = ((state.absmax, torch.uint8), (second.absmax, torch.float32),
+                   (second.code, torch.float32), (offset, torch.float32))
+        if state.quant_type != "nf4" or state.blocksize != 64 or state.dtype != torch.float16 \
+                or not state.nested or second.blocksize != 256 \
+                or second.dtype != torch.float32 or getattr(second, "nested", False):
+            return None
+    except (AttributeError, TypeError, ValueError):
+        return None
+    if not isinstance(shape, (tuple, list)) or type(n) is not int or type(k) is not int \
+            or n <= 0 or k <= 0 or not isinstance(packed, torch.Tensor):
+        return None
+    device = packed.device
+    if device.type != "cuda" or packed.dtype != torch.uint8 or not packed.is_contiguous() \
+            or packed.ndim not in (1, 2) or packed.numel() * 2 < n * k:
+        return None
+    blocks = cdiv(n * k, 64)
+    for (t, dtype), least in zip(buffers, (blocks, cdiv(blocks, 256), 256, 1)):
+        if not isinstance(t, torch.Tensor) or t.dtype != dtype or t.device != device \
+                or not t.is_contiguous() or t.requires_grad or t.numel() < least:
+            return None
+    return (n, k) if offset.numel() == 1 else None
+
+
 def _validate_state(packed, state, out_dtype):
     """Return the (N, K) shape of a supported nested NF4 state, else raise ValueError."""
+    if out_dtype == torch.float16:
+        shape = _accepted(packed, state)
+        if shape is not None:
+            return shape
     enforce(NESTED_STATE_RULES, packed=packed, state=state, out_dtype=out_dtype)
     return _matrix_shape(state)
 

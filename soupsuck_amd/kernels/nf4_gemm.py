@@ -21,6 +21,7 @@ from torch.autograd.function import once_differentiable
 
 from .. import _lib
 from ..contract import Rule, enforce
+from ..native import nodes
 from .nf4 import _validate_state
 
 
@@ -182,3 +183,16 @@ class NF4Linear(torch.autograd.Function):
         (packed,) = ctx.saved_tensors
         dx = nf4_matmul(grad.contiguous(), packed, ctx.state, transpose=True)
         return dx, None, None, None
+
+
+def nf4_linear(x, packed, state, bias=None):
+    """NF4Linear on the native node; the Python node where K or the codes' alignment need the
+    decode-then-dense path, or while timing hooks are installed."""
+    n, k = _validate_state(packed, state, torch.float16)
+    enforce(MATMUL_RULES, x=x, packed=packed, bias=bias, transpose=False, width_in=k, width_out=n)
+    native = nodes() if _fused_ok(packed, k) else None
+    if native is None:
+        return NF4Linear.apply(x, packed, state, bias)
+    second = state.state2
+    return native.nf4_linear(x, packed, state.absmax, second.absmax, second.code, state.offset,
+                             n, k, bias)

@@ -39,6 +39,7 @@ from torch.autograd.function import once_differentiable
 from . import _lib
 from .kernels.nf4 import _validate_state
 from .kernels.nf4_gemm import gemm_f16, nf4_dx_2d, nf4_forward_2d
+from .native import nodes
 
 
 def _nf4_args(packed, state):
@@ -310,6 +311,21 @@ class _QLoRAProjection(torch.autograd.Function):
                 None, None, None, None, None, None)
 
 
+def _fused_node(x, lora_a, lora_b, packed, state, bias, scaling, nf4, dropout):
+    """_QLoRAFused on the native node (the Python one while timing hooks are installed).  The
+    node keeps the workspaces of the stream it is issued on, where its backward runs too."""
+    native = nodes()
+    if native is None:
+        return _QLoRAFused.apply(x, lora_a, lora_b, packed, state, bias, scaling, nf4, dropout)
+    n, k, _ = nf4
+    t, dev = x.numel() // k, x.device
+    stream = _lib.stream(dev)
+    second = state.state2
+    return native.qlora(x, lora_a, lora_b, packed, state.absmax, second.absmax, second.code,
+                        state.offset, n, k, bias, scaling, dropout,
+                        _gemm_ws(t, n, k, dev, stream)[0], _qlora_rank_ws(t, n, k, dev, stream))
+
+
 def qlora_projection(x, lora_a, lora_b, packed, state, bias=None, scaling=2.0, dropout_p=0.0,
                      training=True):
     """out = X . Wdec^T + bias + scaling * (drop(X) . A^T) . B^T with NF4 W (fp16 compute)."""
@@ -331,12 +347,11 @@ def qlora_projection(x, lora_a, lora_b, packed, state, bias=None, scaling=2.0, d
     active = dropout_p > 0.0 and training
     with _on_device(x.device):
         if fused and not active:
-            return _QLoRAFused.apply(x, lora_a, lora_b, packed, state, bias, float(scaling), nf4,
-                                     None)
+            return _fused_node(x, lora_a, lora_b, packed, state, bias, float(scaling), nf4, None)
         # The fused dropout's seed is a kernel argument: a HIP graph would replay one mask
         # forever, so under capture the mask comes from torch's graph-safe generator.
         if fused and x.data_ptr() % 16 == 0 and not torch.cuda.is_current_stream_capturing():
-            return _QLoRAFused.apply(x, lora_a, lora_b, packed, state, bias, float(scaling), nf4,
-                                     (dropout_seed(), float(dropout_p)))
+            return _fused_node(x, lora_a, lora_b, packed, state, bias, float(scaling), nf4,
+                               (dropout_seed(), float(dropout_p)))
         return _QLoRAProjection.apply(x, lora_a, lora_b, packed, state, bias, float(scaling),
                                       float(dropout_p), bool(training))

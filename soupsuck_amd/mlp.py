@@ -81,20 +81,26 @@ def _projections(mlp):
     return None if any(p is None for p in parts) else parts
 
 
-def eligible_mlp(mlp, x):
-    """Frozen bias-free NF4 gate/up/down of matching shapes on x's device, SiLU, CUDA fp16/fp32 x."""
+def _eligible_parts(mlp, x):
+    """The three projections (_nf4) when the MLP is eligible for x, else None."""
     if not isinstance(x, torch.Tensor) or not x.is_cuda or x.dtype not in (torch.float16,
                                                                           torch.float32):
-        return False
+        return None
     act = getattr(getattr(mlp, "config", None), "hidden_act", "silu")
     if act != "silu":
-        return False
+        return None
     parts = _projections(mlp)
     if parts is None:
-        return False
+        return None
     (_, _, ng, kg), (_, _, nu, ku), (_, _, nd, kd) = parts
-    return (kg == ku == nd == x.shape[-1] and ng == nu == kd
+    fits = (kg == ku == nd == x.shape[-1] and ng == nu == kd
             and all(p[0].device == x.device for p in parts))
+    return parts if fits else None
+
+
+def eligible_mlp(mlp, x):
+    """Frozen bias-free NF4 gate/up/down of matching shapes on x's device, SiLU, CUDA fp16/fp32 x."""
+    return _eligible_parts(mlp, x) is not None
 
 
 def _workspace(t, n, k, device):
@@ -417,7 +423,8 @@ def prepare_mlp_offload(model, max_rows=2048):
 
 def fused_qwen2_mlp(mlp, x, recompute=None, offload=None):
     """Run an eligible frozen NF4 MLP; raise ValueError otherwise (solution/mlp.py:579-612)."""
-    if not eligible_mlp(mlp, x):
+    parts = _eligible_parts(mlp, x)
+    if parts is None:
         raise ValueError("Expected frozen bias-free fp16 NF4 Linear4bit projections on CUDA")
     if recompute is None:
         recompute = os.environ.get("SOUP_MLP_RECOMPUTE") == "1" or _recompute_layer(mlp)
@@ -431,7 +438,7 @@ def fused_qwen2_mlp(mlp, x, recompute=None, offload=None):
         if not torch.is_grad_enabled() or not x.requires_grad:
             shape = x.shape
             x2d = x.reshape(-1, shape[-1]).to(torch.float16).contiguous()
-            out, _, _ = mlp_forward_2d(x2d, _projections(mlp), keep=False)
+            out, _, _ = mlp_forward_2d(x2d, parts, keep=False)
             return out.reshape(*shape[:-1], out.shape[-1]).to(x.dtype)
         return _FrozenMLP.apply(x, mlp, bool(recompute), offload)
 
