@@ -30,9 +30,9 @@ Kept logits: when the fp16 logits [N, V] fit KEEP_LOGITS_BUDGET (1 GiB; 251 MB
 at configs[3]) and a backward may run, the forward's products write into one
 [N, V] buffer and the backward reads the logits from there (rows picked through
 the labelled-row indices) instead of recomputing h . W_c^T: one product per
-chunk fewer.  The forward's products then span several chunks (as many as fill
-one wave of 256 x 256 output tiles: two at configs[3]) and one statistics launch
-follows them all; its pieces are those of a chunk-by-chunk forward, so the
+chunk fewer.  The forward's product then spans the whole vocabulary of an fp16 head
+(several chunks of any other head, _product_span) and one statistics launch follows;
+its pieces are those of a chunk-by-chunk forward, so the
 outputs are the same bits.  The backward's
 steps span as many chunks as DERIVATIVE_BUDGET holds of dz and dz' (the whole
 vocabulary at configs[3]): one derivative launch and two long products.  Above
@@ -98,12 +98,17 @@ def _gather_rows(src, index, out=None):
 _CUS = {}
 
 
-def _product_span(rows, chunk, dev):
-    """Vocabulary columns per logits product when the forward keeps its logits: whole
-    chunks, as many as fit one wave of 256 x 256 output tiles on the device's CUs (T =
-    826: two chunks of 8192, 256 tiles, against 224 tiles of 128 x 256 for one chunk).
-    The statistics pieces do not change, and an output element does not depend on the
-    product's width, so the results are the same bits."""
+def _product_span(rows, chunk, weight):
+    """Vocabulary columns per logits product when the forward keeps its logits.  An fp16
+    head is read in place, by one product over the whole vocabulary while it is inside the
+    kernel's 32-bit offsets (T = 826, 151936 x 1536: 453 us, against 503 us for ten
+    products of two chunks, each ending in a wave of tiles that leaves CUs idle).  Other
+    heads are converted piece by piece: whole chunks, as many as fit one wave of 256 x 256
+    output tiles on the device's CUs.  The statistics pieces do not change, and an output
+    element does not depend on the product's width, so the results are the same bits."""
+    vocab, dev = weight.shape[0], weight.device
+    if weight.dtype == torch.float16 and weight.is_contiguous() and 2 * weight.numel() < 1 << 31:
+        return vocab
     if dev not in _CUS:
         _CUS[dev] = torch.cuda.get_device_properties(dev).multi_processor_count
     tiles = -(-rows // 256) * -(-chunk // 256)
@@ -152,7 +157,7 @@ def _forward(hidden16, weight, targets, ignore_index, chunk, keep):
                   start // chunk * per_chunk, slots, ignore_index, stream)
 
     if keep:
-        for start, width in _vocab_chunks(vocab, _product_span(rows, chunk, dev)):
+        for start, width in _vocab_chunks(vocab, _product_span(rows, chunk, weight)):
             gemm_f16(hidden16, _head_rows(weight, start, width), b_trans=True,
                      out=tile[:, start:start + width])
         # Every logit at hand: one statistics launch when the pieces tile whole chunks
