@@ -15,18 +15,32 @@
 // k-steps: k-step j takes k 32 g + 8 j .. + 7 from every lane group g.  The
 // MFMA sums over its 32 k in any order, so X is read with the same
 // permutation: lane (r, g) supplies X[m + r][32 g + 8 j .. + 7].
-// Every load an iteration consumes -- weight runs and X -- is issued PF
-// iterations ahead into a register ring (statically indexed by unrolling),
-// which keeps tens of KB of weight reads in flight per CU.  X is small and
-// L2-resident: for up to two 16-row M tiles each lane loads its 64-byte X
-// fragment runs directly (no LDS, no barrier: the waves of a workgroup run
-// independently); for more M tiles X is shared through a double-buffered LDS
-// tile whose 272-byte row pitch keeps the 16-row fragment reads
-// bank-conflict-free.
+// Up to 32 rows (nf4_skinny_fwd_kernel): every load an iteration consumes --
+// weight runs and X -- is issued PF iterations ahead into a register ring
+// (statically indexed by unrolling), and each lane loads its 64-byte X fragment
+// runs directly (no LDS, no barrier: the waves of a workgroup run
+// independently).
+//
+// 33 .. 128 rows (nf4_skinny_lds_kernel): X is shared through a double-buffered
+// LDS tile whose 272-byte row pitch keeps the 16-row fragment reads
+// bank-conflict-free.  Decoding a k-step takes as many VALU cycles as its MFMAs
+// take matrix cycles, so the two are software-pipelined within the wave: while
+// k-step j multiplies, j + 1 is scaled and rounded and the table reads of j + 2
+// are in flight (decode first, multiply after left each pipe idle in turn).
+// One instance per 16 rows: 101 rows multiply 7 tiles, not 8.
 //
 // K is split over grid.y; every split writes fp32 partials [split][T][N] and
 // the split-K reduce applies the epilogue (bias, LoRA add) with the GEMM's
-// rounding order.
+// rounding order.  Each split is at least four 128-deep iterations long above 32 rows:
+// shorter ones fill the chip but write and reduce an fp32 plane for every 256 k.
+//
+// Kernel and reduce on MI355X, us, before (one instance for 65 .. 128 rows, decode ahead
+// of the MFMAs, splits of two iterations) -> after, [N, K] at T = 40, 64, 101, 128:
+// [3584, 18944] 30.7, 29.9, 38.1, 39.2 -> 26.9, 27.8, 35.0, 37.9; [3584, 3584] 16.1, 18.8,
+// 22.8, 23.0 -> 11.9, 13.6, 17.5, 19.9; [1536, 8960] 21.7, 23.7, 27.3, 27.3 -> 13.7, 15.4,
+// 18.7, 19.5; [8960, 1536] 15.8, 17.8, 22.9, 24.2 -> 12.3, 14.1, 18.3, 20.4.  At least 3 or
+// 6 iterations: [1536, 8960] at 101 rows 20.2 or 19.3.  A bank-conflict-free table (one
+// copy of the 16 values per lane, one read per code) costs 5% more than the pair table.
 
 #include "gemm.h"
 
@@ -38,26 +52,24 @@ constexpr int kSkPitch = kSkK + 8; // LDS row pitch of the X tile (halves)
 constexpr int kSkNB = 2;           // 16-row weight blocks per wave
 constexpr int kSkRowsPerWG = 4 * kSkNB * 16;
 
-// Everything one iteration consumes, loaded kPF iterations ahead: the weight
-// runs (codes, qabs byte, absmax2) and the X data -- direct path: the lane's
-// 64-byte X fragment run per M tile; LDS path: the thread's X tile chunks.
+// Everything one iteration consumes, loaded PF iterations ahead: the weight
+// runs (codes, qabs byte, absmax2) and the lane's 64-byte X fragment run per M tile.
 // Because no load is consumed soon after it is issued, the in-order load
 // counter never forces the ring's newer loads to complete early.
-template <int MT, bool XLDS>
+template <int MT>
 struct Slot {
-  static constexpr int kX = XLDS ? MT : MT * 4;
+  static constexpr int kX = MT * 4;
   u32x4 codes[kSkNB];
   uint32_t q[kSkNB];
   float a2[kSkNB];
   u32x4 x[kX];
 };
 
-template <int MT, bool XLDS, int PF>
+template <int MT, int PF>
 __global__ __launch_bounds__(256, 2) void nf4_skinny_fwd_kernel(
     const half_t* __restrict__ x, int64_t ldx, int64_t t, Nf4View w, int64_t n, int64_t k,
     int64_t k_split, float* __restrict__ part) {
-  using SlotT = Slot<MT, XLDS>;
-  __shared__ __attribute__((aligned(16))) half_t sx[XLDS ? 2 : 1][XLDS ? MT * 16 * kSkPitch : 8];
+  using SlotT = Slot<MT>;
   __shared__ float s_code2[256];
   // Both NF4 values of a code byte in one LDS read: {NF4[e >> 4], NF4[e & 15]}.
   __shared__ __attribute__((aligned(8))) float2 s_pair[256];
@@ -87,17 +99,10 @@ __global__ __launch_bounds__(256, 2) void nf4_skinny_fwd_kernel(
   const half_t* xsrc[SlotT::kX];
 #pragma unroll
   for (int i = 0; i < SlotT::kX; ++i) {
-    if constexpr (XLDS) {
-      const int c = tid + 256 * i;  // X tile chunk: row c / 16, 16-byte chunk c % 16
-      int64_t row = c >> 4;
-      row = row < t ? row : t - 1;
-      xsrc[i] = x + row * ldx + kbeg + (c & 15) * 8;
-    } else {
-      const int mt = i >> 2, j = i & 3;  // lane's run X[mt*16 + r][32 g + 8 j ..]
-      int64_t row = mt * 16 + r16;
-      row = row < t ? row : t - 1;
-      xsrc[i] = x + row * ldx + kbeg + 32 * g + 8 * j;
-    }
+    const int mt = i >> 2, j = i & 3;  // lane's run X[mt*16 + r][32 g + 8 j ..]
+    int64_t row = mt * 16 + r16;
+    row = row < t ? row : t - 1;
+    xsrc[i] = x + row * ldx + kbeg + 32 * g + 8 * j;
   }
   auto fetch = [&](int it, SlotT& sl) {
 #pragma unroll
@@ -132,21 +137,6 @@ __global__ __launch_bounds__(256, 2) void nf4_skinny_fwd_kernel(
   __syncthreads();  // code tables visible
 
   auto step = [&](int it, SlotT& sl, bool refill) {
-    if constexpr (XLDS) {
-      // Publish this iteration's X tile (double buffered: the barrier of the
-      // previous iteration ordered every wave's reads of this buffer from two
-      // iterations ago before this write).
-      const int buf = it & 1;
-#pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const int c = tid + 256 * i;
-        *reinterpret_cast<u32x4*>(&sx[buf][(c >> 4) * kSkPitch + (c & 15) * 8]) = sl.x[i];
-      }
-      // LDS-only barrier: __syncthreads() would also wait for every
-      // outstanding global load, i.e. drain the prefetch ring.
-      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this thread's LDS writes done
-      asm volatile("s_barrier" ::: "memory");
-    }
     half8 bfrag[kSkNB][4];
 #pragma unroll
     for (int nb = 0; nb < kSkNB; ++nb) {
@@ -172,12 +162,7 @@ __global__ __launch_bounds__(256, 2) void nf4_skinny_fwd_kernel(
       half8 af[MT];
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
-        if constexpr (XLDS) {
-          af[mt] = *reinterpret_cast<const half8*>(
-              &sx[it & 1][(mt * 16 + r16) * kSkPitch + 32 * g + 8 * j]);
-        } else {
-          af[mt] = __builtin_bit_cast(half8, sl.x[mt * 4 + j]);
-        }
+        af[mt] = __builtin_bit_cast(half8, sl.x[mt * 4 + j]);
       }
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
@@ -221,16 +206,192 @@ __global__ __launch_bounds__(256, 2) void nf4_skinny_fwd_kernel(
   }
 }
 
+// 33 .. 128 rows: X shared by the workgroup's waves through LDS.
+template <int MT>
+__global__ __launch_bounds__(256, 2) void nf4_skinny_lds_kernel(
+    const half_t* __restrict__ x, int64_t ldx, int64_t t, Nf4View w, int64_t n, int64_t k,
+    int64_t k_split, float* __restrict__ part) {
+  constexpr int kSkRing = MT == 8 ? 2 : 3;  // iterations of codes in flight (registers)
+  struct Codes {
+    u32x4 codes[kSkNB];
+    uint32_t q[kSkNB];
+    float a2[kSkNB];
+  };
+  __shared__ __attribute__((aligned(16))) half_t sx[2][MT * 16 * kSkPitch];
+  __shared__ float s_code2[256];
+  // Both NF4 values of a code byte in one LDS read: {NF4[e >> 4], NF4[e & 15]}.
+  __shared__ __attribute__((aligned(8))) float2 s_pair[256];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  const int r16 = lane & 15;
+  const int g = lane >> 4;
+  const int64_t kbeg = (int64_t)blockIdx.y * k_split;
+  const int64_t klen = k - kbeg < k_split ? k - kbeg : k_split;
+  const int iters = (int)(klen / kSkK);
+  const int last = iters - 1;
+  const int64_t wrow0 = (int64_t)blockIdx.x * kSkRowsPerWG + wave * kSkNB * 16;
+
+  // Weight rows past N and X rows past T are clamped (their outputs are never stored).
+  int64_t code_elem[kSkNB];
+#pragma unroll
+  for (int nb = 0; nb < kSkNB; ++nb) {
+    int64_t row = wrow0 + nb * 16 + r16;
+    row = row < n ? row : n - 1;
+    code_elem[nb] = row * k + kbeg + 32 * g;
+  }
+  // X tile chunk c = tid + 256 i: row c / 16, 16-byte chunk c % 16.  Only the last 16-row
+  // tile can reach past T.
+  const int64_t tail_row = (tid >> 4) + 16 * (MT - 1) < t ? (tid >> 4) + 16 * (MT - 1) : t - 1;
+  const half_t* const x_first = x + (tid >> 4) * ldx + kbeg + (tid & 15) * 8;
+  const half_t* const x_tail = x + tail_row * ldx + kbeg + (tid & 15) * 8;
+  Codes ring[kSkRing];
+  u32x4 xr[MT];
+  auto fetch_codes = [&](int it, Codes& sl) {
+    it = it < last ? it : last;
+#pragma unroll
+    for (int nb = 0; nb < kSkNB; ++nb) {
+      const int64_t e = code_elem[nb] + (int64_t)it * kSkK;
+      const int64_t block = e >> 6;
+      sl.codes[nb] = *reinterpret_cast<const u32x4*>(w.packed + (e >> 1));
+      sl.q[nb] = w.qabs[block];
+      sl.a2[nb] = w.absmax2[block >> 8];
+    }
+  };
+  auto fetch_x = [&](int it) {
+    const int64_t at = (int64_t)(it < last ? it : last) * kSkK;
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+      xr[i] = *reinterpret_cast<const u32x4*>((i < MT - 1 ? x_first + i * 16 * ldx : x_tail) + at);
+  };
+
+  const float c2 = w.code2[tid];
+  const float offset = w.offset[0];
+  fetch_codes(0, ring[0]);
+  fetch_x(0);
+#pragma unroll
+  for (int s = 1; s < kSkRing; ++s) fetch_codes(s, ring[s]);
+  s_code2[tid] = c2;
+  s_pair[tid] = float2{kNF4[tid >> 4], kNF4[tid & 15]};
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+  asm volatile("s_barrier" ::: "memory");
+
+  float2 pr[kSkNB][4];
+  half8 bc[kSkNB];
+  float sc[kSkNB];
+  auto lookup = [&](const Codes& sl, int j) {
+#pragma unroll
+    for (int nb = 0; nb < kSkNB; ++nb)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) pr[nb][b] = s_pair[(sl.codes[nb][j] >> (8 * b)) & 0xffu];
+  };
+  auto convert = [&](half8 (&b8)[kSkNB]) {
+#pragma unroll
+    for (int nb = 0; nb < kSkNB; ++nb)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        b8[nb][2 * b] = f32_to_f16(pr[nb][b].x * sc[nb]);
+        b8[nb][2 * b + 1] = f32_to_f16(pr[nb][b].y * sc[nb]);
+      }
+  };
+  auto scales = [&](const Codes& sl) {
+#pragma unroll
+    for (int nb = 0; nb < kSkNB; ++nb) sc[nb] = s_code2[sl.q[nb]] * sl.a2[nb] + offset;
+  };
+
+  float4v acc[MT][kSkNB];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nb = 0; nb < kSkNB; ++nb) acc[mt][nb] = float4v{0.f, 0.f, 0.f, 0.f};
+
+  // Pipeline over k-steps: while the MFMAs of one run, the next one's weights are scaled
+  // and rounded and the table reads of the one after are in flight.
+  scales(ring[0]);
+  lookup(ring[0], 0);
+  convert(bc);
+  lookup(ring[0], 1);
+  auto step = [&](int it, Codes& cur, const Codes& next) {
+    const int buf = it & 1;
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+      *reinterpret_cast<u32x4*>(&sx[buf][((tid >> 4) + 16 * i) * kSkPitch + (tid & 15) * 8]) =
+          xr[i];
+    // LDS-only barrier: __syncthreads() would drain the loads in flight.  The barrier of
+    // the previous iteration ordered every wave's reads of this buffer before the writes.
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this thread's LDS writes done
+    asm volatile("s_barrier" ::: "memory");
+    fetch_x(it + 1);
+    const half_t* const tile = &sx[buf][r16 * kSkPitch + 32 * g];
+    half8 af[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+      af[mt] = *reinterpret_cast<const half8*>(tile + mt * 16 * kSkPitch);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      half8 bn[kSkNB];
+      if (j == 3) scales(next);
+      convert(bn);
+      lookup(j < 2 ? cur : next, j < 2 ? j + 2 : j - 2);
+      if (j == 1) fetch_codes(it + kSkRing, cur);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+        for (int nb = 0; nb < kSkNB; ++nb)
+          acc[mt][nb] =
+              __builtin_amdgcn_mfma_f32_16x16x32_f16(af[mt], bc[nb], acc[mt][nb], 0, 0, 0);
+        if (j < 3)
+          af[mt] = *reinterpret_cast<const half8*>(tile + mt * 16 * kSkPitch + 8 * (j + 1));
+      }
+#pragma unroll
+      for (int i = 0; i < MT * kSkNB; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                     // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                     // LDS read
+        __builtin_amdgcn_sched_group_barrier(0x002, 80 / (MT * kSkNB), 0);     // VALU
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int nb = 0; nb < kSkNB; ++nb) bc[nb] = bn[nb];
+    }
+  };
+  int it0 = 0;
+  for (; it0 + kSkRing <= iters; it0 += kSkRing) {
+#pragma unroll
+    for (int s = 0; s < kSkRing; ++s) step(it0 + s, ring[s], ring[(s + 1) % kSkRing]);
+  }
+#pragma unroll
+  for (int s = 0; s < kSkRing - 1; ++s)
+    if (it0 + s < iters) step(it0 + s, ring[s], ring[s + 1]);
+
+  // Partials: lane holds D[4 g + r][r16] of each 16x16 (rows = X rows, cols = weight rows).
+  float* out = part + (int64_t)blockIdx.y * t * n;
+#pragma unroll
+  for (int nb = 0; nb < kSkNB; ++nb) {
+    const int64_t col = wrow0 + nb * 16 + r16;
+    if (col >= n) continue;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t row = mt * 16 + 4 * g + r;
+        if (row < t) out[row * n + col] = acc[mt][nb][r];
+      }
+  }
+}
+
 }  // namespace
 
 SkinnyPlan skinny_plan(int64_t t, int64_t n, int64_t k) {
   SkinnyPlan plan{0, 0, 0};
   if (t <= 0 || t > kSkinnyMaxT || n <= 0 || k <= 0 || k % kSkK != 0) return plan;
-  plan.mt = t <= 16 ? 1 : t <= 32 ? 2 : t <= 64 ? 4 : 8;
-  // About two workgroups per CU, each split at least two iterations long.
+  plan.mt = (int)cdiv(t, 16);
+  // About two workgroups per CU, each split at least two iterations long, or four where
+  // the partial planes are tall (above 32 rows; measured at the top of the file).
   const int64_t cols = cdiv(n, kSkRowsPerWG);
   int64_t s = 512 / cols;
-  if (s > k / (2 * kSkK)) s = k / (2 * kSkK);
+  const int64_t least = plan.mt > 2 ? 4 : 2;
+  if (s > k / (least * kSkK)) s = k / (least * kSkK);
   if (s < 1) s = 1;
   plan.k_split = cdiv(cdiv(k, s), kSkK) * kSkK;
   plan.splits = cdiv(k, plan.k_split);
@@ -256,21 +417,27 @@ int nf4_skinny_fwd(const GemmParams& p, int epi, void* partials, size_t partial_
   const dim3 grid((unsigned)cdiv(p.N, kSkRowsPerWG), (unsigned)plan.splits);
   switch (plan.mt) {
     case 1:
-      hipLaunchKernelGGL((nf4_skinny_fwd_kernel<1, false, 4>), grid, dim3(256), 0, stream, p.A,
+      hipLaunchKernelGGL((nf4_skinny_fwd_kernel<1, 4>), grid, dim3(256), 0, stream, p.A,
                          p.lda, p.M, p.w, p.N, p.K, plan.k_split, part);
       break;
     case 2:
-      hipLaunchKernelGGL((nf4_skinny_fwd_kernel<2, false, 3>), grid, dim3(256), 0, stream, p.A,
+      hipLaunchKernelGGL((nf4_skinny_fwd_kernel<2, 3>), grid, dim3(256), 0, stream, p.A,
                          p.lda, p.M, p.w, p.N, p.K, plan.k_split, part);
       break;
-    case 4:
-      hipLaunchKernelGGL((nf4_skinny_fwd_kernel<4, true, 4>), grid, dim3(256), 0, stream, p.A,
-                         p.lda, p.M, p.w, p.N, p.K, plan.k_split, part);
-      break;
+#define SS_SKINNY(MT)                                                                        \
+  case MT:                                                                                   \
+    hipLaunchKernelGGL((nf4_skinny_lds_kernel<MT>), grid, dim3(256), 0, stream, p.A, p.lda,  \
+                       p.M, p.w, p.N, p.K, plan.k_split, part);                              \
+    break;
+    SS_SKINNY(3)
+    SS_SKINNY(4)
+    SS_SKINNY(5)
+    SS_SKINNY(6)
+    SS_SKINNY(7)
+    SS_SKINNY(8)
+#undef SS_SKINNY
     default:
-      hipLaunchKernelGGL((nf4_skinny_fwd_kernel<8, true, 2>), grid, dim3(256), 0, stream, p.A,
-                         p.lda, p.M, p.w, p.N, p.K, plan.k_split, part);
-      break;
+      return SS_ERR_UNSUPPORTED;
   }
   SS_CHECK_LAUNCH("nf4_skinny_fwd_kernel");
   GemmParams q = p;
