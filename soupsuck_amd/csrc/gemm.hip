@@ -1103,7 +1103,8 @@ static int qlora_backward(const char* fn, const uint16_t* dy, int64_t lddy, int6
   // in disjoint exchange areas (dB after dZ's, dA after dB's) and counter
   // ranges, where both fill CUs the GEMM leaves idle instead of lengthening
   // the preparation launch (measured at T = 990: k / v backward 18.0 -> 14.8
-  // us, q / o 32 -> 30); next to a split-K reduce it gained nothing (the
+  // us, q / o 32 -> 30; the tiles that take a whole CU run both in a launch of
+  // their own, gemm_nt); next to a split-K reduce it gained nothing (the
   // reduce grew by what the preparation launch lost), so there it stays in
   // the preparation launch.
   bool vda = false, vdb = false;

@@ -599,7 +599,15 @@ int dispatch_nt(const GemmParams& p, int cfg, int64_t splits, hipStream_t stream
   } else {
     if (layout) return SS_ERR_UNSUPPORTED;
   }
-  switch (cfg) {
+  if constexpr (EPI == EPI_GLU) {
+    switch (cfg) {
+      case 1: return launch_nt<Nt64, CT, EPI>(p, splits, stream);
+      case 2: return launch_nt<Nt128x64, CT, EPI>(p, splits, stream);
+      case 3: return launch_nt<Nt128, CT, EPI>(p, splits, stream);
+      case 8: return launch_nt<NtPingPong, CT, EPI>(p, splits, stream);
+      default: return SS_ERR_UNSUPPORTED;
+    }
+  } else switch (cfg) {
     case 1: return launch_nt<Nt64, CT, EPI>(p, splits, stream);
     case 2: return launch_nt<Nt128x64, CT, EPI>(p, splits, stream);
     case 3: return launch_nt<Nt128, CT, EPI>(p, splits, stream);
@@ -794,7 +802,15 @@ int gemm_nt(const GemmParams& p0, int ct, int epi, hipStream_t stream, void* par
       SS_CHECK_LAUNCH("rank_tail_kernel");
       return SS_OK;
     }
-    if (p.glu) return dispatch_nt<SS_F16, EPI_GLU>(p, plan.cfg, 1, stream);
+    // The SwiGLU epilogue moves three more planes through the tile's waves: on the four
+    // waves of the wide tiles it outlasts what their loop gains (frozen MLP at T = 990,
+    // 1536 x 8960, both activations in epilogues: 435 us on 256 x 160 tiles, 323 us so), so the
+    // eight waves of the ping-pong tile do it there, or 128 x 128 tiles where few would run.
+    if (p.glu) {
+      int cfg = plan.cfg;
+      if (cfg > 3) cfg = cdiv(p.M, 256) * cdiv(p.N, 256) >= device_cu_count() / 2 ? 8 : 3;
+      return dispatch_nt<SS_F16, EPI_GLU>(p, cfg, 1, stream);
+    }
     return dispatch_nt<SS_F16, EPI_PLAIN>(p, plan.cfg, 1, stream);
   }
   return dispatch_nt<SS_F32, EPI_PLAIN>(p, plan.cfg, 1, stream);
