@@ -259,10 +259,12 @@ struct TileReader {
   }
 };
 
-// Scores whose register row (8 (r / 4) + r % 4) is below lo or from hi on become -inf.
+// Scores whose register row (8 (r / 4) + r % 4) is below lo or from hi on become -inf (and
+// their statistics, if given, 0).
 // Called under a rarely true uniform branch; the ties keep the compares and selects
 // inside it (hoisted, they were 32 of the ~90 vector instructions of every half tile).
-__device__ __forceinline__ void mask_rows(float16v& s, int lo, int hi) {
+template <class... Stats>
+__device__ __forceinline__ void mask_rows(float16v& s, int lo, int hi, Stats&... stats) {
   tie(lo);
   tie(hi);
 #pragma unroll
@@ -270,7 +272,9 @@ __device__ __forceinline__ void mask_rows(float16v& s, int lo, int hi) {
     float x = s[r];
     tie(x);
     const int row = 8 * (r >> 2) + (r & 3);
-    s[r] = row < lo || row >= hi ? -INFINITY : x;
+    const bool masked = row < lo || row >= hi;
+    s[r] = masked ? -INFINITY : x;
+    ((stats[r] = masked ? 0.f : stats[r]), ...);
   }
 }
 
@@ -703,10 +707,11 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attn_bwd_dkdv_kernel(AttnArgs 
     dv[dt] = float16v{};
   }
 
-  auto mask = [&](float16v& s, int qs) {
-    if (qs < k0w + 31 || qs + 32 > len) {  // the diagonal or the row's end
-      mask_rows(s, mykey - qs - 4 * h, len - qs - 4 * h);
-    }
+  // A masked entry is P = 0 whatever its query's statistic is: a query with a NaN score has
+  // a NaN lse, which keys that it does not attend to must not see (exp2(-inf - 0) instead).
+  auto mask = [&](float16v& s, float (&lse)[16], int qs) {
+    if (qs < k0w + 31 || qs + 32 > len)  // the diagonal or the row's end
+      mask_rows(s, mykey - qs - 4 * h, len - qs - 4 * h, lse);
   };
   // P and dS of elements 2 k and 2 k + 1.
   auto elements = [&](const float16v& s, const float16v& dp, const float (&lse)[16],
@@ -762,7 +767,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attn_bwd_dkdv_kernel(AttnArgs 
               dv[st % 4] = mfma(operand(p[b][st / 4]), f, dv[st % 4]);
           } else if constexpr (i & 1) {
             e[b] = mfma(f, vf[st], e[b]);
-            if constexpr (st == 7) mask(s[b], qt + 32 * (h0 + b));
+            if constexpr (st == 7) mask(s[b], lse[b], qt + 32 * (h0 + b));
           } else {
             s[b] = mfma(f, kf[st], st == 0 ? float16v{} : s[b]);
           }

@@ -59,3 +59,41 @@ def test_block_edges(device, lengths, hq, hk, scale):
         norm = np.linalg.norm(ref_g)
         err = np.linalg.norm(_np(x).astype(np.float64) - ref_g)
         assert err <= 1e-2 * norm, f"d{name}: {err:.3e} of {norm:.3e}"
+
+
+@pytest.mark.parametrize("lengths,hq,hk", [
+    ((45, 100), 2, 1),             # 64-token blocks
+    ((130, 300), 2, 2),            # 64-token blocks, dK / dV written directly
+    ((450,) * 10, 16, 16),         # 128-token blocks
+])
+def test_nan_query_reaches_only_what_it_attends_to(device, lengths, hq, hk):
+    """A query row of NaN (head 0, token 10 of every packed row) makes its own output and dQ NaN
+    and, as its P, dV of the keys it attends to; no other row of O, dQ or dV."""
+    t = sum(lengths)
+    print(f"case NaN rows={len(lengths)} T={t} hq={hq} hk={hk}", flush=True)
+    gen = torch.Generator().manual_seed(t)
+
+    def heads(h):
+        x = torch.randn((1, t, h * 128), generator=gen).half().to(device)
+        return x.view(1, t, h, 128).transpose(1, 2)
+
+    q, k, v = heads(hq), heads(hk), heads(hk)
+    starts = np.cumsum((0,) + lengths[:-1])
+    for s in starts:
+        q[0, 0, s + 10] = float("nan")
+    q, k, v = (x.requires_grad_() for x in (q, k, v))
+    o = packed_causal_attention(q, k, v, lengths, 128 ** -0.5)
+    g = torch.randn((1, t, hq, 128), generator=gen).half().to(device)
+    dq, _, dv = torch.autograd.grad(o, (q, k, v), g)
+
+    def bad(x):   # [heads, tokens]
+        return ~torch.isfinite(x.detach()).all(-1)[0].cpu().numpy()
+
+    own = np.zeros((hq, t), bool)
+    own[0, starts + 10] = True
+    seen = np.zeros((hk, t), bool)
+    for s in starts:
+        seen[0, s:s + 11] = True
+    np.testing.assert_array_equal(bad(o.transpose(1, 2)), own)
+    np.testing.assert_array_equal(bad(dq), own)
+    np.testing.assert_array_equal(bad(dv), seen)
