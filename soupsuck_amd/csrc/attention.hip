@@ -181,8 +181,9 @@ __device__ __forceinline__ void dma4_at(const void* p, uint32_t lds) {
 // Loads of one operand's tiles: DMA g (of 16) brings rows 4 g .. 4 g + 3, a wave
 // issues four of them.  A whole tile takes wave-uniform row addresses and four
 // lane offsets kept in registers; a tile past the packed row's end (or a token
-// stride whose offsets need 64 bits) takes an address per lane, rows past the end
-// re-reading the last row (their scores are masked, or their results not stored).
+// stride that is negative or whose offsets need 64 bits: they are unsigned 32-bit bytes)
+// takes an address per lane, rows past the end re-reading the last row (their scores are
+// masked, or their results not stored).
 struct TileLoader {
   static constexpr int kPer = 16 / kWaves;  // DMAs per wave and tile
   const half_t* base;  // first token of the row, this head
@@ -200,7 +201,7 @@ struct TileLoader {
     return (lane & 15) ^ ((lane >> 4) << 2) ^ j;
   }
   __device__ __forceinline__ void issue(int t0, uint32_t lds, int wave) const {
-    if (t0 + kTile <= len && tok < (1 << 28)) {
+    if (t0 + kTile <= len && tok >= 0 && tok < (1 << 28)) {
       const half_t* rows = base + (int64_t)(t0 + 4 * wave * kPer) * tok;
 #pragma unroll
       for (int j = 0; j < kPer; ++j)

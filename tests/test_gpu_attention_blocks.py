@@ -16,6 +16,7 @@ import pytest
 import torch
 
 from oracle import attention as oattn
+from soupsuck_amd import _lib
 from soupsuck_amd.kernels.attention import packed_causal_attention
 
 pytestmark = pytest.mark.gpu
@@ -97,3 +98,40 @@ def test_nan_query_reaches_only_what_it_attends_to(device, lengths, hq, hk):
     np.testing.assert_array_equal(bad(o.transpose(1, 2)), own)
     np.testing.assert_array_equal(bad(dq), own)
     np.testing.assert_array_equal(bad(dv), seen)
+
+
+@pytest.mark.parametrize("lengths,hq,hk", [((130, 65), 2, 1), ((700,) * 6, 16, 16)])
+def test_reversed_token_axis(device, lengths, hq, hk):
+    """The C entry points take any token stride: operands stored last token first (a negative
+    stride from the last row) give the bits of the same operands stored forwards."""
+    t = sum(lengths)
+    print(f"case reversed rows={len(lengths)} T={t} hq={hq} hk={hk}", flush=True)
+    gen = torch.Generator().manual_seed(t)
+    cu = torch.tensor(np.cumsum((0,) + lengths), dtype=torch.int32, device=device)
+    q, dout = (torch.randn((t, hq, 128), generator=gen).half().to(device) for _ in range(2))
+    k, v = (torch.randn((t, hk, 128), generator=gen).half().to(device) for _ in range(2))
+    size = _lib.load().ss_attn_varlen_bwd_workspace_size(hq, hk, t)
+    ws = torch.empty(size, dtype=torch.uint8, device=device)
+    stream = _lib.stream(device)
+
+    def run(reverse):
+        def operand(x):
+            held = x.flip(0).contiguous() if reverse else x
+            first = held[-1] if reverse else held[0]
+            return held, (first.data_ptr(), -x.stride(0) if reverse else x.stride(0), x.stride(1))
+
+        ins = [operand(x) for x in (q, k, v)]
+        args = sum((a for _, a in ins), ())
+        o, ovec = operand(torch.empty_like(q))
+        lse = torch.empty((hq, t), device=device)
+        sizes = (cu.data_ptr(), len(lengths), max(lengths), t, hq, hk, 128, 128 ** -0.5)
+        _lib.call("ss_attn_varlen_fwd", *args, *sizes, *ovec, lse.data_ptr(), stream)
+        g, gvec = operand(dout)
+        outs = [operand(torch.empty_like(x)) for x in (q, k, v)]
+        _lib.call("ss_attn_varlen_bwd", *args, *ovec, *gvec, lse.data_ptr(), *sizes,
+                  *sum((a for _, a in outs), ()), ws.data_ptr(), size, stream)
+        torch.cuda.synchronize()
+        return [x.flip(0) if reverse else x for x in (o, *(held for held, _ in outs))] + [lse]
+
+    for got, want in zip(run(True), run(False)):
+        assert torch.equal(got, want)
