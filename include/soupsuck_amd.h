@@ -93,8 +93,8 @@ int ss_nf4_gemm_fwd(const uint16_t* x, int64_t ldx, int64_t t, const uint8_t* pa
  * tight serving loops, harnesses that forbid hipMalloc).  Same arguments,
  * result and kernels as ss_nf4_gemm_fwd (bit-identical output); its scratch is
  * a fixed 64 MiB device array per GPU, held until the process ends.  Shapes
- * whose forward needs more scratch than that (T >= 256 with a large weight)
- * are rejected with SS_ERR_INVALID_ARGUMENT; every T < 256 at the Qwen2.5
+ * whose forward needs more scratch than that (T >= 256 with a decoded weight of
+ * more than 64 MiB) are rejected with SS_ERR_INVALID_ARGUMENT; every T < 256 at the Qwen2.5
  * 1.5B/7B projection shapes fits.  Nothing is allocated and no library routine
  * that allocates is called.  Calls that overlap in time on one GPU share the
  * scratch and race: issue them on one stream, or serialise them. */

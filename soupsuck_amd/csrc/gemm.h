@@ -268,9 +268,9 @@ __device__ __forceinline__ void epilogue_f16(const GemmParams& p, int64_t row, i
 // Dense NT GEMM (A [M,K] and B [N,K] both K-contiguous fp16) on the
 // direct-to-LDS pipelined kernel.  Returns SS_ERR_UNSUPPORTED (nothing
 // launched) when the operands do not meet its requirements: 16-byte aligned
-// rows and K % 64 == 0.  `partials` (may be null) is scratch for split-K:
-// long-K products with few output tiles are split over k when it holds
-// nt_partial_bytes(M, N, K) bytes.
+// rows and K % 64 == 0.  `partials` (may be null) is scratch for split-K: the
+// product takes the best plan whose planes fit it (nt_partial_bytes(M, N, K)
+// bytes hold those of the best one).
 int gemm_nt(const GemmParams& p, int ct, int epi, hipStream_t stream, void* partials = nullptr,
             size_t partial_bytes = 0);
 // LDS-staged fp16 epilogue switch of the NT and fused NF4 launchers (default on).
@@ -279,12 +279,13 @@ bool staged_epilogue_enabled();
 // the fp32 partial planes and an fp16 plane for a LoRA forward's rank term.
 size_t nt_partial_bytes(int64_t m, int64_t n, int64_t k, int layout = 0);
 // Tile configuration (1..8 in gemm_nt.hip's list) and split-K plan of an
-// M x N x K product on the NT kernels (layout: bit 0 / 1 for K-major A / B).
+// M x N x K product on the NT kernels (layout: bit 0 / 1 for K-major A / B), with
+// split-K planes of at most `scratch` bytes.
 struct NtPlan {
   int cfg;
   int64_t splits, k_split;
 };
-NtPlan nt_plan(int64_t m, int64_t n, int64_t k, int layout = 0);
+NtPlan nt_plan(int64_t m, int64_t n, int64_t k, int layout = 0, size_t scratch = SIZE_MAX);
 
 // Fused NF4 forward (gemm_nf4.hip): Y = X . Wdec^T with p.M = T, p.N = N,
 // p.K = K, p.A = X, p.w = the NF4 weight, the NT kernel's tile plan and

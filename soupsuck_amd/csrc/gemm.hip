@@ -526,6 +526,9 @@ static bool aligned16(const void* ptr, int64_t ld) {
 
 using namespace ss;
 
+// Scratch of ss_nf4_gemm_fwd_noalloc.
+constexpr size_t kNoAllocScratchBytes = size_t(64) << 20;
+
 // Decode-first workspace: the fp16 weight (forward [N,K], backward its
 // transpose), rounded up to 256 bytes, followed by the fp32 split-K partials
 // of the dense product when it is split.
@@ -677,9 +680,14 @@ static int run_fwd(GemmParams& p, void* workspace, size_t workspace_bytes, hipSt
     p.ldb = k;
     p.b_vec = 1;
     const size_t dec = decoded_bytes(n, k);
-    void* part = workspace_bytes > dec ? static_cast<char*>(workspace) + dec : nullptr;
-    return dispatch<OP_ROW, OP_ROW, SS_F16, EPI>(p, s, "gemm_kernel<f16 nt>", part,
-                                                 part ? workspace_bytes - dec : 0);
+    // The split planes stay within what ss_nf4_gemm_fwd_noalloc has beside a weight that fits
+    // its scratch, so that both entry points take one plan and give the same bits (1536 x
+    // 8960 at T = 2689 .. 3072 is not split in two for it: 88 us either way).
+    size_t room = workspace_bytes > dec ? workspace_bytes - dec : 0;
+    if (EPI == EPI_PLAIN && dec <= kNoAllocScratchBytes && room > kNoAllocScratchBytes - dec)
+      room = kNoAllocScratchBytes - dec;
+    void* part = room ? static_cast<char*>(workspace) + dec : nullptr;
+    return dispatch<OP_ROW, OP_ROW, SS_F16, EPI>(p, s, "gemm_kernel<f16 nt>", part, room);
   }
   return dispatch<OP_ROW, OP_NF4_ROW, SS_F16, EPI>(p, s, "gemm_kernel<nf4 fwd>");
 }
@@ -786,7 +794,6 @@ extern "C" int ss_nf4_gemm_fwd(const uint16_t* x, int64_t ldx, int64_t t, const 
 // array and race.
 namespace {
 
-constexpr size_t kNoAllocScratchBytes = size_t(64) << 20;
 __device__ __align__(256) static unsigned char scratch[kNoAllocScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -836,17 +843,20 @@ extern "C" int ss_nf4_gemm_fwd_noalloc(const uint16_t* x, int64_t ldx, int64_t t
   SS_CHECK_ARG(ldx >= k && ldy >= n, "%s: leading dimensions too small", fn);
   // The streaming, skinny and fused kernels read X with 16-byte loads.  An X they cannot
   // take sends run_fwd to the decode-first path, as ss_nf4_gemm_fwd with its full
-  // workspace does, so the scratch must then hold the decoded weight and the dense
-  // product's partials; sizing it for the fast paths alone would fall through to the
-  // in-loop decoder, a different kernel.
+  // workspace does, so the scratch must then hold the decoded weight; sizing it for the
+  // fast paths alone would fall through to the in-loop decoder, a different kernel.  The
+  // dense product after the decode splits K as far as the rest of the scratch goes.
   const bool x_vec = reinterpret_cast<uintptr_t>(x) % 16 == 0 && ldx % 8 == 0;
-  const size_t need = x_vec ? fwd_workspace_bytes(t, n, k)
+  const size_t full = x_vec ? fwd_workspace_bytes(t, n, k)
                             : decoded_bytes(n, k) + ss::nt_partial_bytes(t, n, k);
-  SS_CHECK_ARG(need <= kNoAllocScratchBytes,
+  const size_t least =
+      x_vec && t < decode_first_threshold() ? full : decoded_bytes(n, k);
+  SS_CHECK_ARG(least <= kNoAllocScratchBytes,
                "%s: T=%lld N=%lld K=%lld needs %zu bytes of scratch, more than the fixed "
                "%zu-byte device scratch of this entry point; use ss_nf4_gemm_fwd with a "
                "workspace of ss_nf4_gemm_workspace_size() bytes",
-               fn, (long long)t, (long long)n, (long long)k, need, kNoAllocScratchBytes);
+               fn, (long long)t, (long long)n, (long long)k, least, kNoAllocScratchBytes);
+  const size_t need = full < kNoAllocScratchBytes ? full : kNoAllocScratchBytes;
   void* ws = nullptr;
   if (need) {
     rc = scratch_on_current_device(fn, &ws);
@@ -1118,7 +1128,9 @@ static int qlora_backward(const char* fn, const uint16_t* dy, int64_t lddy, int6
   if (vda) {
     p.tail_blocks = da_blocks;
     p.tail_ran = &da_ran;
-    if (vdb && nt_plan(t, k, n).splits == 1) {
+    const size_t dec = decoded_bytes(n, k);
+    const size_t scratch = workspace && workspace_bytes > dec ? workspace_bytes - dec : 0;
+    if (vdb && nt_plan(t, k, n, 0, scratch).splits == 1) {
       p.tail2 = dbg;
       p.tail2_blocks = db_blocks;
       pj.grad_blocks = 0;

@@ -634,6 +634,15 @@ bool aligned16(const void* ptr) { return reinterpret_cast<uintptr_t>(ptr) % 16 =
 
 }  // namespace
 
+// Split-K scratch: the fp32 partial planes, then (256-byte aligned) the fp16
+// LoRA plane of a split LoRA forward.
+static size_t nt_plane_offset(int64_t m, int64_t n, int64_t splits) {
+  return ((size_t)(splits * m * n) * sizeof(float) + 255) / 256 * 256;
+}
+static size_t nt_split_bytes(int64_t m, int64_t n, int64_t splits) {
+  return nt_plane_offset(m, n, splits) + (size_t)(m * n) * sizeof(half_t);
+}
+
 // Configuration and split-K plan for an M x N x K product: the cheapest by a cost model
 // of the time a launch takes,
 //   start + q (tile + stages (stage + load f)),   q = ceil(workgroups / CUs),
@@ -658,8 +667,10 @@ constexpr TileCost kTileCosts[] = {
     {7, 256, 256, 0.0f, 13.1f, 0.896f, 0.532f},
 };
 
-// layout: bit 0 / 1 for K-major A / B (GemmParams::a_t, b_t).
-NtPlan nt_plan(int64_t m, int64_t n, int64_t k, int layout) {
+// layout: bit 0 / 1 for K-major A / B (GemmParams::a_t, b_t).  scratch: what the planes of
+// a split may take; without room for them the tile is the best one for an unsplit product
+// (990 x 1536 x 8960: 45 us on 128x64 tiles, 77 us on the 128x256 tiles of the 5-way split).
+NtPlan nt_plan(int64_t m, int64_t n, int64_t k, int layout, size_t scratch) {
   const int64_t cus = device_cu_count();
   NtPlan plan{1, 1, k};
   if ((layout & 1) && cdiv(m, 256) * cdiv(n, 256) >= cus / 2) {
@@ -677,6 +688,7 @@ NtPlan nt_plan(int64_t m, int64_t n, int64_t k, int layout) {
     for (int64_t s = 1; s <= most; ++s) {
       const int64_t k_split = cdiv(cdiv(k, s), 64) * 64;
       if (cdiv(k, k_split) != s) continue;
+      if (s > 1 && nt_split_bytes(m, n, s) > scratch) break;
       const int64_t q = cdiv(tiles * s, cus);
       const float f = (float)(tiles * s) / (float)(q * cus);
       const float stages = (float)(k_split / 64);
@@ -701,15 +713,6 @@ int splitk_reduce(const GemmParams& p, int splits, int ct, int epi, hipStream_t 
   if (epi == EPI_RANK) return reduce_nt<SS_F16, EPI_RANK>(p, splits, stream);
   if (p.glu) return reduce_nt<SS_F16, EPI_GLU>(p, splits, stream);
   return reduce_nt<SS_F16, EPI_PLAIN>(p, splits, stream);
-}
-
-// Split-K scratch: the fp32 partial planes, then (256-byte aligned) the fp16
-// LoRA plane of a split LoRA forward.
-static size_t nt_plane_offset(int64_t m, int64_t n, int64_t splits) {
-  return ((size_t)(splits * m * n) * sizeof(float) + 255) / 256 * 256;
-}
-static size_t nt_split_bytes(int64_t m, int64_t n, int64_t splits) {
-  return nt_plane_offset(m, n, splits) + (size_t)(m * n) * sizeof(half_t);
 }
 
 size_t nt_partial_bytes(int64_t m, int64_t n, int64_t k, int layout) {
@@ -742,13 +745,8 @@ int gemm_nt(const GemmParams& p0, int ct, int epi, hipStream_t stream, void* par
   if (epi != EPI_PLAIN && (!aligned16(p.lz) || (epi == EPI_LORA && !aligned16(p.lb))))
     return SS_ERR_UNSUPPORTED;
   if (ct != SS_F16 && epi != EPI_PLAIN) return SS_ERR_UNSUPPORTED;
-  NtPlan plan = nt_plan(p.M, p.N, p.K, (p.a_t ? 1 : 0) | (p.b_t ? 2 : 0));
-  const size_t need = nt_split_bytes(p.M, p.N, plan.splits);
-  if (plan.splits > 1 && (!partials || partial_bytes < need ||
-                          reinterpret_cast<uintptr_t>(partials) % 16 != 0)) {
-    plan.splits = 1;
-    plan.k_split = p.K;
-  }
+  const NtPlan plan = nt_plan(p.M, p.N, p.K, (p.a_t ? 1 : 0) | (p.b_t ? 2 : 0),
+                              partials && aligned16(partials) ? partial_bytes : 0);
   // The rank-16 grad tail rides on unsplit dX products (rank-16 epilogue) after the GEMM
   // tiles where the tile's LDS lets two or more workgroups share a CU (64 columns: it
   // fills CUs that the GEMM leaves idle; q / o / k / v backward 6-11 us faster).  Behind

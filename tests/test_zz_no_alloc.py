@@ -5,7 +5,8 @@ device array instead of a caller workspace, so at every shape its output must
 be bit-identical to ss_nf4_gemm_fwd's (a stronger bar than the GEMM tolerance:
 the same kernels run on the same operands).  Cases cover every forward path
 the scratch serves: streaming (T <= 32), skinny (T <= 128), the fused NF4 GEMM
-(128 < T < 256) and decode-first (T >= 256, small weight).  Two calls run back
+(128 < T < 256) and decode-first (T >= 256, small weight; the dense product splits K only
+as far as its planes fit beside the decoded weight).  Two calls run back
 to back with nothing between them, the second on a smaller input, so the
 second call meets the first call's leftovers in the shared scratch.  A shape
 whose forward needs more scratch than the array holds is rejected with
@@ -27,6 +28,9 @@ CASES = [
     ((8960, 1536), (200, 100)),   # fused, then skinny
     ((1536, 1536), (990, 300)),   # decode-first (decoded weight in the scratch), twice
     ((512, 3584), (32, 1)),       # streaming, twice
+    ((1536, 8960), (2689, 300)),  # decode-first beside planes of a split that would not fit
+    ((1536, 8960), (3072, 700)),
+    ((2048, 8192), (2304, 2056)),
 ]
 
 
