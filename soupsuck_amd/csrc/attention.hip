@@ -41,7 +41,8 @@
 // run along the token axis) take different banks too.
 //
 // Workgroups: 4 waves on 128 queries (keys) of one head, 32 per wave; batches too small
-// to fill the chip that way take 64, two waves for each 32 (short_batch).
+// to fill the chip that way take 64, two waves for each 32 (short_batch).  Batches of short
+// rows take 16-row waves (attention_rows16.h).
 //
 // Backward: a dQ kernel per (row, query block, q head), which also writes
 // delta = rowsum(dO . O); then a dK / dV kernel per (row, key block, q head)
@@ -832,6 +833,14 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attn_bwd_dkdv_kernel(AttnArgs 
   }
 }
 
+}  // namespace
+}  // namespace ss
+
+#include "attention_rows16.h"
+
+namespace ss {
+namespace {
+
 // dK / dV of a GQA group: the q heads' fp32 partials added in head order
 // (deterministic), dK scaled; four consecutive d per thread.
 __global__ __launch_bounds__(256) void attn_bwd_reduce_kernel(AttnArgs a, const float* part_k,
@@ -857,6 +866,33 @@ __global__ __launch_bounds__(256) void attn_bwd_reduce_kernel(AttnArgs a, const 
   }
   *reinterpret_cast<half4*>(a.dk + t * a.dk_tok + (int64_t)kvh * a.dk_head + d) = ok;
   *reinterpret_cast<half4*>(a.dv + t * a.dv_tok + (int64_t)kvh * a.dv_head + d) = ov;
+}
+
+// Batches that the 16-row waves (attention_rows16.h) run faster, per step, by their longest
+// row; us on 16-row against the better 32-row kernel, 12 q / 2 kv heads:
+//   forward, 48: 4000 tokens in rows of 16 23.7 / 28.3, of 32 15.9 / 16.4, 2000 in rows of 48 7.4 /
+//     10.5 (4000 14.0 / 12.7), 4000 in rows of 64 13.9 / 12.1;
+//   dQ, 64: rows of 16 31.0 / 37.2, of 48 17.4 / 17.9, of 64 16.5 / 16.4 (16 / 16 heads 19.8 /
+//     22.5), of 100 19.8 / 15.7;
+//   dK / dV, 192: rows of 16 32.6 / 65, of 64 20.2 / 26.6, of 100 28.2 / 25.3 (at 1000 tokens 12.5 /
+//     14.4), of 158 29.0 / 30.4 (7900 tokens 47.4 / 56.5), of 300 38.1 / 32.5;
+// and rows up to 128 while 64-token blocks are at most 5/4 of the CUs, where the time is
+// one workgroup's latency (300 tokens in rows of 100: forward 6.8 / 7.1, dQ 7.3 / 8.2; 1000 in
+// rows of 100: dQ 7.6 / 9.9; 2000 11.8 / 12.3).
+bool few_blocks(int64_t total, int hq) {
+  return cdiv(total, kBlk) * hq * 4 <= 5 * (int64_t)device_cu_count();
+}
+bool rows16_fwd(int max_len, int64_t total, int hq) {
+  return max_len <= 48 || (max_len <= 128 && few_blocks(total, hq));
+}
+bool rows16_dq(int max_len, int64_t total, int hq) {
+  return max_len <= 64 || (max_len <= 128 && few_blocks(total, hq));
+}
+bool rows16_dkdv(int max_len) { return max_len <= 192; }
+
+// Grid of the 16-row kernels.
+dim3 rows16_grid(const AttnArgs& a, int max_len) {
+  return dim3((unsigned)cdiv(max_len, kBlk), (unsigned)a.hq, (unsigned)a.rows);
 }
 
 // Blocks of 64 queries / keys with two waves for each 32 (<2, 2>) when blocks of 128
@@ -924,7 +960,9 @@ extern "C" int ss_attn_varlen_fwd(const void* q, int64_t q_tok, int64_t q_head, 
   a.span = small ? 64 : 128;
   a.blocks = (int)cdiv(max_len, a.span);
   hipStream_t st = (hipStream_t)stream;
-  if (small)
+  if (rows16_fwd(max_len, total, hq))
+    hipLaunchKernelGGL(attn_fwd_rows16_kernel, rows16_grid(a, max_len), dim3(256), 0, st, a);
+  else if (small)
     hipLaunchKernelGGL((attn_fwd_kernel<2, 2>), item_grid(a), dim3(256), 0, st, a);
   else
     hipLaunchKernelGGL((attn_fwd_kernel<4, 1>), item_grid(a), dim3(256), 0, st, a);
@@ -986,12 +1024,17 @@ extern "C" int ss_attn_varlen_bwd(const void* q, int64_t q_tok, int64_t q_head, 
   a.span = small ? 64 : 128;
   a.blocks = (int)cdiv(max_len, a.span);
   hipStream_t st = (hipStream_t)stream;
-  if (small)
+  if (rows16_dq(max_len, total, hq))
+    hipLaunchKernelGGL(attn_bwd_dq_rows16_kernel, rows16_grid(a, max_len), dim3(256), 0, st, a);
+  else if (small)
     hipLaunchKernelGGL((attn_bwd_dq_kernel<2, 2>), item_grid(a), dim3(256), 0, st, a);
   else
     hipLaunchKernelGGL((attn_bwd_dq_kernel<4, 1>), item_grid(a), dim3(256), 0, st, a);
   SS_CHECK_LAUNCH("attn_bwd_dq_kernel");
-  if (small)
+  if (rows16_dkdv(max_len))
+    hipLaunchKernelGGL(attn_bwd_dkdv_rows16_kernel, rows16_grid(a, max_len), dim3(256), 0, st, a,
+                       part_k, part_v);
+  else if (small)
     hipLaunchKernelGGL((attn_bwd_dkdv_kernel<2, 2>), item_grid(a), dim3(256), 0, st, a, part_k,
                        part_v);
   else

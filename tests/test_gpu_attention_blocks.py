@@ -1,7 +1,7 @@
 """GPU parity of the attention kernels at the edges of their blocks and variants.
 
 The kernels work in blocks of 128 queries / keys (64 for batches too small to fill
-the chip), 64-token tiles and 32-token halves, and find their (block, row) from the row
+the chip and, on 16-row waves, for batches of short rows), 64-token tiles and 32-token halves, and find their (block, row) from the row
 lengths (at most 64 rows) or from the grid (more rows).  Each case puts row ends on
 both sides of those edges, for both block sizes, with and without GQA, and with the
 signs of the softmax scale that the kernels treat apart.
@@ -37,6 +37,16 @@ def _np(t):
     (MANY, 60, 10, 128 ** -0.5),    # positions from the grid, 128-token blocks
     ((40, 300), 4, 2, -0.07),
     ((40, 300), 4, 2, 0.0),
+    # 16-row waves: all three steps, dQ and dK / dV, dK / dV alone, none; and few tokens
+    ((1, 15, 16, 17, 31, 32) * 20, 12, 2, 128 ** -0.5),
+    ((32, 33, 48, 47) * 10, 12, 12, 128 ** -0.5),
+    ((32, 33, 48, 63, 64) * 10, 12, 12, 128 ** -0.5),
+    ((64, 65, 127, 129, 191, 192) * 3, 12, 2, 128 ** -0.5),
+    ((64, 65, 127, 129, 193) * 3, 12, 2, 128 ** -0.5),
+    ((128, 65, 1), 12, 2, 128 ** -0.5),
+    ((128, 129, 1), 12, 2, 128 ** -0.5),
+    ((20, 32), 4, 2, -0.07),
+    ((20, 32), 4, 2, 0.0),
 ])
 def test_block_edges(device, lengths, hq, hk, scale):
     t = sum(lengths)
@@ -63,7 +73,8 @@ def test_block_edges(device, lengths, hq, hk, scale):
 
 
 @pytest.mark.parametrize("lengths,hq,hk", [
-    ((45, 100), 2, 1),             # 64-token blocks
+    ((45, 100), 2, 1),             # 16-row waves
+    ((45, 200), 2, 1),             # 64-token blocks
     ((130, 300), 2, 2),            # 64-token blocks, dK / dV written directly
     ((450,) * 10, 16, 16),         # 128-token blocks
 ])
@@ -100,7 +111,8 @@ def test_nan_query_reaches_only_what_it_attends_to(device, lengths, hq, hk):
     np.testing.assert_array_equal(bad(dv), seen)
 
 
-@pytest.mark.parametrize("lengths,hq,hk", [((130, 65), 2, 1), ((700,) * 6, 16, 16)])
+@pytest.mark.parametrize("lengths,hq,hk", [((50, 65), 2, 1), ((230, 65), 2, 1),
+                                                 ((700,) * 6, 16, 16)])
 def test_reversed_token_axis(device, lengths, hq, hk):
     """The C entry points take any token stride: operands stored last token first (a negative
     stride from the last row) give the bits of the same operands stored forwards."""
