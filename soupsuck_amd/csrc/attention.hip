@@ -895,10 +895,16 @@ dim3 rows16_grid(const AttnArgs& a, int max_len) {
   return dim3((unsigned)cdiv(max_len, kBlk), (unsigned)a.hq, (unsigned)a.rows);
 }
 
-// Blocks of 64 queries / keys with two waves for each 32 (<2, 2>) when blocks of 128
-// would be fewer than two per CU: such a batch is a latency chain per workgroup.
-bool short_batch(int64_t total, int hq) {
-  return cdiv(total, 128) * hq < 2 * (int64_t)device_cu_count();
+// Blocks of 64 queries / keys with two waves for each 32 (<2, 2>) while such blocks (a row's
+// last one half full) number at most 3/2 of the CUs, 2 of them for long rows, whose blocks
+// are long chains of tiles; beyond that the chip is full and 128-token blocks read each
+// tile for twice the rows.  Forward + backward, us, <2, 2> against <4, 1>: 12 q / 2 kv heads, rows
+// of 300: 1500 tokens 50.0 / 49.8, 3000 80.1 / 64.4; rows of 1000: 2000 tokens 82.8 / 96.3, 3000
+// 107.4 / 105.9, 4000 134.5 / 117.4; 16 / 16 heads, rows of 300: 1500 tokens 52.0 / 46.0, 3000 94.1 /
+// 72.9, 3900 117.3 / 92.4; 28 / 4 heads, 1000 in rows of 500 66.4 / 67.6, one row of 1000 88.5 / 96.9.
+bool short_batch(int64_t total, int rows, int max_len, int hq) {
+  const int64_t blocks = (total / 64 + rows / 2) * hq;
+  return blocks * 2 <= (max_len < 768 ? 3 : 4) * (int64_t)device_cu_count();
 }
 
 // Grid of the items (Item): all (block, row) positions, or with few rows as many as
@@ -956,7 +962,7 @@ extern "C" int ss_attn_varlen_fwd(const void* q, int64_t q_tok, int64_t q_head, 
   a.out = (half_t*)o; a.out_tok = o_tok; a.out_head = o_head;
   a.lse2 = lse2; a.cu = cu_seqlens; a.total = total; a.hq = hq; a.hk = hk; a.scale = scale;
   a.rows = rows;
-  const bool small = short_batch(total, hq);
+  const bool small = short_batch(total, rows, max_len, hq);
   a.span = small ? 64 : 128;
   a.blocks = (int)cdiv(max_len, a.span);
   hipStream_t st = (hipStream_t)stream;
@@ -1020,7 +1026,7 @@ extern "C" int ss_attn_varlen_bwd(const void* q, int64_t q_tok, int64_t q_head, 
   float* part_k = hq == hk ? nullptr : reinterpret_cast<float*>(base);
   float* part_v = hq == hk ? nullptr : reinterpret_cast<float*>(base + part);
   a.rows = rows;
-  const bool small = short_batch(total, hq);
+  const bool small = short_batch(total, rows, max_len, hq);
   a.span = small ? 64 : 128;
   a.blocks = (int)cdiv(max_len, a.span);
   hipStream_t st = (hipStream_t)stream;
