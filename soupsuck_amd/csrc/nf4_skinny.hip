@@ -31,8 +31,8 @@
 //
 // K is split over grid.y; every split writes fp32 partials [split][T][N] and
 // the split-K reduce applies the epilogue (bias, LoRA add) with the GEMM's
-// rounding order.  Each split is at least four 128-deep iterations long above 32 rows:
-// shorter ones fill the chip but write and reduce an fp32 plane for every 256 k.
+// rounding order.  Above 32 rows a split is mostly at least four 128-deep iterations long:
+// shorter ones fill the chip but write and reduce an fp32 plane for every 256 k (skinny_plan).
 //
 // Kernel and reduce on MI355X, us, before (one instance for 65 .. 128 rows, decode ahead
 // of the MFMAs, splits of two iterations) -> after, [N, K] at T = 40, 64, 101, 128:
@@ -386,11 +386,20 @@ SkinnyPlan skinny_plan(int64_t t, int64_t n, int64_t k) {
   SkinnyPlan plan{0, 0, 0};
   if (t <= 0 || t > kSkinnyMaxT || n <= 0 || k <= 0 || k % kSkK != 0) return plan;
   plan.mt = (int)cdiv(t, 16);
-  // About two workgroups per CU, each split at least two iterations long, or four where
-  // the partial planes are tall (above 32 rows; measured at the top of the file).
+  // About two workgroups per CU, each split at least two iterations long.  Four above 32
+  // rows, where the partial planes are tall (measured at the top of the file), unless that
+  // leaves a short K's chain to few workgroups: K of at most 2560, half the CUs idle and
+  // planes of at most 8 MB.  Kernel and reduce, us, [N, K] with two / four iterations at T = 33,
+  // 64, 128: [256, 1536] 7.2 / 9.0, 7.9 / 9.8, 10.3 / 12.7; [896, 2304] 8.0 / 9.7, 9.1 / 10.8, 12.3 /
+  // 14.4; [4096, 1536] 8.9 / 9.6, 11.0 / 11.4, 16.5 / 15.8; [8192, 1024] 9.5 / 10.2, 12.4 / 11.9, 20.2 /
+  // 17.1; [18944, 512] 11.4 / 10.5, 15.1 / 12.8, 22.3 / 18.4; [1024, 4096] 10.6 / 9.8, 12.3 / 11.0,
+  // 15.8 / 14.6.
   const int64_t cols = cdiv(n, kSkRowsPerWG);
   int64_t s = 512 / cols;
-  const int64_t least = plan.mt > 2 ? 4 : 2;
+  int64_t least = 2;
+  if (plan.mt > 2 && (k > 20 * kSkK || cols * (k / (4 * kSkK)) > 128 ||
+                      k / (2 * kSkK) * n * t > 2 << 20))
+    least = 4;
   if (s > k / (least * kSkK)) s = k / (least * kSkK);
   if (s < 1) s = 1;
   plan.k_split = cdiv(cdiv(k, s), kSkK) * kSkK;

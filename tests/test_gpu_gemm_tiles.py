@@ -21,9 +21,10 @@ def _gate(actual, expected, what):
     assert ok, f"{what}: max_abs={max_abs:.3e} rel_l2={rel:.3e}"
 
 
-# K = 128 k: one iteration (the code ring longer than the work), two, a ring and a bit, and
-# enough for several splits with a shorter last one; N around the 128-row workgroup.
-@pytest.mark.parametrize("n,k", [(40, 128), (128, 256), (136, 640), (64, 2432)])
+# K = 128 k: one iteration (the code ring longer than the work), two, splits of two
+# iterations with a shorter last one, and of four (K above 2560) with a shorter last one; N
+# around the 128-row workgroup.
+@pytest.mark.parametrize("n,k", [(40, 128), (128, 256), (136, 640), (64, 2432), (136, 2944)])
 @pytest.mark.parametrize("t", [33, 48, 49, 64, 65, 81, 96, 101, 112, 113, 128])
 def test_skinny_rows(device, t, n, k):
     state = onf4.quantize_nested(random_weight(n, k, 11))
