@@ -502,7 +502,6 @@ __global__ __launch_bounds__(C::kThreads, C::MINW) void gemm_nf4t_kernel(GemmPar
 #pragma unroll
     for (int j = 0; j < C::FN; ++j) acc[i][j] = float16v{};
   nf4k_mainloop<C, CD>(p, m0, n0, kbeg, klen, smem, acc);
-  static_assert(!GluStage<C>::kOk || GluStage<C>::kBytes <= Nf4Layout<C>::kSmem, "stage");
   nt_epilogue<C, CT, EPI>(p, m0, n0, acc, smem, split);
 }
 
@@ -528,7 +527,6 @@ __global__ __launch_bounds__(C::kThreads, C::MINW) void gemm_nf4_kernel(GemmPara
 #pragma unroll
     for (int j = 0; j < C::FN; ++j) acc[i][j] = float16v{};
   nf4_mainloop<C, CD>(p, m0, n0, kbeg, klen, smem, acc);
-  static_assert(!GluStage<C>::kOk || GluStage<C>::kBytes <= Nf4Layout<C>::kSmem, "stage");
   nt_epilogue<C, CT, EPI>(p, m0, n0, acc, smem, split);
 }
 

@@ -393,7 +393,6 @@ __global__ __launch_bounds__(C::kThreads, C::MINW) void gemm_nt_kernel(GemmParam
   } else {
     nt_mainloop_pp<C, L>(p, m0, n0, kbeg, klen, smem, acc);
   }
-  static_assert(!GluStage<C>::kOk || GluStage<C>::kBytes <= nt_smem_bytes<C, EPI>(), "stage");
   nt_epilogue<C, CT, EPI>(p, m0, n0, acc, smem, split);
 }
 

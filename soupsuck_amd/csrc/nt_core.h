@@ -379,7 +379,7 @@ __device__ __forceinline__ void load_bias(const GemmParams& p, int64_t n0, int w
 // product takes ~1.5 us less; a SwiGLU reading that output next takes ~1.4
 // us more (it no longer finds it in the last-level cache), and the whole
 // decoder layer measured 0.4-1 % faster with them.
-template <class C, int EPI>
+template <class C, int EPI, int SMEM>
 __device__ __forceinline__ void nt_epilogue_staged(const GemmParams& p, int64_t m0, int64_t n0,
                                                    const NtAcc<C>& acc, unsigned char* smem) {
   using G = GluStage<C>;
@@ -398,10 +398,11 @@ __device__ __forceinline__ void nt_epilogue_staged(const GemmParams& p, int64_t 
   load_bias<C>(p, n0, wn, lr, bias);
   wait_vm<0>();
   __syncthreads();
-  // One pass over the whole tile where the ring has room for it, else a pass per wave row
-  // group (whose waves then convert while the others wait).
+  // One pass over the whole tile where the kernel's LDS has room for it, else a pass per wave
+  // row group (whose waves then convert while the others wait).
   constexpr int kGroups = C::BM / C::WM;
-  constexpr bool kWhole = kGroups * G::kBytes <= C::STAGES * C::kStageBytes;
+  constexpr bool kWhole = kGroups * G::kBytes <= SMEM;
+  static_assert((kWhole ? kGroups : 1) * G::kBytes <= SMEM, "staged rows");
   constexpr int kPasses = kWhole ? 1 : kGroups;
 #pragma unroll 1
   for (int q = 0; q < kPasses; ++q) {
@@ -450,13 +451,14 @@ __device__ __forceinline__ void nt_epilogue_staged(const GemmParams& p, int64_t 
   }
 }
 
-// `smem`: the kernel's LDS, at least GluStage<C>::kBytes (staged epilogues).
-template <class C, int CT, int EPI>
+// `smem`: the kernel's LDS, SMEM bytes, which the staged epilogues use.
+template <class C, int CT, int EPI, int SMEM>
 __device__ __forceinline__ void nt_epilogue(const GemmParams& p, int64_t m0, int64_t n0,
-                                            const NtAcc<C>& acc, unsigned char* smem = nullptr,
+                                            const NtAcc<C>& acc, unsigned char (&smem)[SMEM],
                                             int64_t split = 0) {
   if constexpr (EPI == EPI_GLU) {
     if constexpr (GluStage<C>::kOk) {
+      static_assert(GluStage<C>::kBytes <= SMEM, "staged rows");
       if (p.glu_vec) {
         nt_glu_epilogue_lds<C>(p, m0, n0, acc, smem);
         return;
@@ -466,8 +468,8 @@ __device__ __forceinline__ void nt_epilogue(const GemmParams& p, int64_t m0, int
     return;
   }
   if constexpr (CT == SS_F16 && EPI != EPI_PARTIAL && GluStage<C>::kOk) {
-    if (p.c_vec && smem) {
-      nt_epilogue_staged<C, EPI>(p, m0, n0, acc, smem);
+    if (p.c_vec) {
+      nt_epilogue_staged<C, EPI, SMEM>(p, m0, n0, acc, smem);
       return;
     }
   }
