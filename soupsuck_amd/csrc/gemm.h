@@ -288,11 +288,12 @@ struct NtPlan {
 NtPlan nt_plan(int64_t m, int64_t n, int64_t k, int layout = 0, size_t scratch = SIZE_MAX);
 
 // Fused NF4 forward (gemm_nf4.hip): Y = X . Wdec^T with p.M = T, p.N = N,
-// p.K = K, p.A = X, p.w = the NF4 weight, the NT kernel's tile plan and
-// epilogues (EPI_PLAIN / EPI_LORA); the weight is decoded into LDS tiles, never
-// written to memory.  `partials` (may be null) holds the split-K planes
-// (nt_partial_bytes).  SS_ERR_UNSUPPORTED (nothing launched) unless
-// gemm_nf4_fwd_ok.
+// p.K = K, p.A = X, p.w = the NF4 weight, the NT kernel's epilogues (EPI_PLAIN /
+// EPI_LORA); the weight is decoded into LDS tiles, never written to memory.
+// `partials` (may be null) holds the split-K planes (nf4_fused_partial_bytes).
+// SS_ERR_UNSUPPORTED (nothing launched) unless gemm_nf4_fwd_ok: at most
+// kNf4FusedMaxT rows (more are faster decoded once, see gemm_nf4_fwd_preferred).
+constexpr int64_t kNf4FusedMaxT = 256;
 bool gemm_nf4_fwd_ok(const GemmParams& p, int epi);
 // Whether the fused kernel is the faster path for this product (tile plan and
 // M tiles; measured).

@@ -646,13 +646,7 @@ static int run_fwd(GemmParams& p, void* workspace, size_t workspace_bytes, hipSt
     const int rc = nf4_skinny_fwd(p, EPI, workspace, workspace_bytes, s);
     if (rc != SS_ERR_UNSUPPORTED) return rc;
   }
-  // With a preparation launch (the QLoRA step) the decode-first path decodes
-  // inside that launch, without one of its own: there the fused kernel is
-  // taken for one or two 128-row tiles only (measured: at T = 990 the q
-  // projection forward takes 34.3 us fused, 31.0 us decode-first).
-  const bool fused_pays = prep ? p.M > kSkinnyMaxT && p.M <= 256
-                               : p.M > kSkinnyMaxT && gemm_nf4_fwd_preferred(p);
-  if (nf4_fused_enabled() && gemm_nf4_fwd_ok(p, EPI) && (nf4_fused_forced() || fused_pays)) {
+  if (nf4_fused_enabled() && gemm_nf4_fwd_ok(p, EPI) && (nf4_fused_forced() || gemm_nf4_fwd_preferred(p))) {
     // The weight is decoded inside the GEMM; the workspace holds split-K
     // partials only.  A deferred preparation launch carries no decode.
     if (fused) {

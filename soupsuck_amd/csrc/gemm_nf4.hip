@@ -10,11 +10,10 @@
 // only in LDS.
 //
 // The A operand (X rows) and the MFMA / epilogue part are those of the dense
-// NT kernel (nt_core.h, same tile configurations, stage depth BK = 32), so a
-// launch computes exactly what the decode-first path computes with the same
-// configuration: identical fp16 B values (the standalone decoder's
-// arithmetic: fp16_rne(fp32(NF4[c]) * fp32(fp32(code2[q] * absmax2) +
-// offset))), identical k order.
+// NT kernel (nt_core.h, stage depth BK = 32), so a split computes exactly what
+// the decode-first path computes over the same k: identical fp16 B values
+// (the standalone decoder's arithmetic: fp16_rne(fp32(NF4[c]) *
+// fp32(fp32(code2[q] * absmax2) + offset))), identical k order.
 //
 // Per stage kt (32 k) each thread owns DPT = BN * 16 / threads code bytes of
 // one weight row (TPR = 16 / DPT threads per row): they come with the row's
@@ -530,10 +529,9 @@ __global__ __launch_bounds__(C::kThreads, C::MINW) void gemm_nf4_kernel(GemmPara
   nt_epilogue<C, CT, EPI>(p, m0, n0, acc, smem, split);
 }
 
-// Configurations (1, 2 and 8 in nf4_plan).
+// Configurations (1 and 2 in nf4_plan).
 using Nf4Small = NtCfg<64, 64, 2, 2, 32, 4, 2>;
 using Nf4Mid = NtCfg<128, 128, 2, 2, 32, 4, 2>;
-using Nf4Big = NtCfg<256, 256, 2, 4, 32, 4, 2>;
 
 template <class C, int CD, int CT, int EPI>
 int launch_nf4(const GemmParams& p, int64_t splits, hipStream_t stream) {
@@ -546,7 +544,6 @@ int launch_nf4(const GemmParams& p, int64_t splits, hipStream_t stream) {
 template <int CT, int EPI>
 int dispatch_nf4(const GemmParams& p, int cfg, int64_t splits, hipStream_t stream) {
   switch (cfg) {
-    case 8: return launch_nf4<Nf4Big, 8, CT, EPI>(p, splits, stream);
     case 2: return launch_nf4<Nf4Mid, 12, CT, EPI>(p, splits, stream);
     default: return launch_nf4<Nf4Small, 12, CT, EPI>(p, splits, stream);
   }
@@ -566,45 +563,10 @@ int dispatch_nf4t(const GemmParams& p, int64_t splits, hipStream_t stream) {
 
 }  // namespace
 
-// Tile plan of the fused kernel.  One or two 128-row tiles, where streaming the
-// weight sets the pace: 64x64 tiles up to 64 rows, 128x128 above, split over
-// k until about 512 workgroups run, each split at least 512 deep.  More rows (only
-// without the decode-first path's scratch): 256x256 tiles once half the CUs get one,
-// 128x128 split over a long K, 64x64 split for a few tiles.
-static NtPlan nf4_wide_plan(int64_t m, int64_t n, int64_t k) {
-  NtPlan plan{1, 1, k};
-  const int64_t t256 = cdiv(m, 256) * cdiv(n, 256);
-  const int64_t t128 = cdiv(m, 128) * cdiv(n, 128);
-  int64_t s = 1;
-  if (t256 >= 96 && cdiv(m, 128) * cdiv(n, 256) <= 256 && k < 8192) {
-    plan.cfg = 2;
-  } else if (t256 >= 128) {
-    plan.cfg = 8;
-  } else if (k >= 32768) {
-    plan.cfg = 8;
-    s = 256 / t256 < k / 2048 ? 256 / t256 : k / 2048;
-  } else if (k >= 2048 && t128 < 256) {
-    plan.cfg = 2;
-    s = 512 / t128 < k / 1024 ? 512 / t128 : k / 1024;
-    if (s > 8) s = 8;
-  } else if (t256 >= 96) {
-    plan.cfg = 8;
-    s = 2;
-  } else if (t128 >= 128) {
-    plan.cfg = 2;
-  } else if (t128 < 64 && k >= 1024) {
-    s = 256 / (cdiv(m, 64) * cdiv(n, 64));
-    if (s > k / 384) s = k / 384;
-    if (s > 8) s = 8;
-  }
-  if (s < 1) s = 1;
-  plan.k_split = cdiv(cdiv(k, s), 64) * 64;
-  plan.splits = cdiv(k, plan.k_split);
-  return plan;
-}
-
+// Tile plan of the fused kernel, which takes at most 256 rows (one or two 128-row tiles), so
+// that streaming the weight sets the pace: 64x64 tiles up to 64 rows, 128x128 above, split
+// over k until about 512 workgroups run, each split at least 512 deep.
 NtPlan nf4_plan(int64_t m, int64_t n, int64_t k) {
-  if (m > 256) return nf4_wide_plan(m, n, k);
   NtPlan plan{m <= 64 ? 1 : 2, 1, k};
   const int64_t bm = plan.cfg == 1 ? 64 : 128;
   const int64_t tiles = cdiv(m, bm) * cdiv(n, bm);
@@ -617,7 +579,7 @@ NtPlan nf4_plan(int64_t m, int64_t n, int64_t k) {
 }
 
 bool gemm_nf4_fwd_ok(const GemmParams& p, int epi) {
-  if (p.M <= 0 || p.N <= 0 || p.K <= 0 || p.K % 64 != 0) return false;
+  if (p.M <= 0 || p.M > kNf4FusedMaxT || p.N <= 0 || p.K <= 0 || p.K % 64 != 0) return false;
   if (reinterpret_cast<uintptr_t>(p.A) % 16 != 0 || p.lda % 8 != 0 ||
       reinterpret_cast<uintptr_t>(p.w.packed) % 8 != 0)
     return false;
@@ -643,11 +605,11 @@ bool gemm_nf4_fwd_ok(const GemmParams& p, int epi) {
 // T <= 128 stays on the streaming / skinny kernels (7B gate at T = 33: 32 vs
 // 48 us fused).
 bool gemm_nf4_fwd_preferred(const GemmParams& p) {
-  return p.M > kSkinnyMaxT && p.M <= 256;
+  return p.M > kSkinnyMaxT && p.M <= kNf4FusedMaxT;
 }
 
 size_t nf4_fused_partial_bytes(int64_t m, int64_t n, int64_t k) {
-  if (m <= 0 || n <= 0 || k <= 0 || k % 64 != 0) return 0;
+  if (m <= 0 || m > kNf4FusedMaxT || n <= 0 || k <= 0 || k % 64 != 0) return 0;
   const NtPlan plan = nf4_plan(m, n, k);
   return plan.splits > 1 ? (size_t)(plan.splits * m * n) * sizeof(float) : 0;
 }

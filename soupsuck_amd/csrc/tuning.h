@@ -28,7 +28,7 @@
 #ifndef SS_TUNE_NF4_STREAM
 #define SS_TUNE_NF4_STREAM 1
 #endif
-// Fused NF4 GEMM: 0 off, 1 where measured faster, 2 wherever it applies.
+// Fused NF4 GEMM: 0 off, 1 where measured faster, 2 wherever it applies (up to 256 rows).
 #ifndef SS_TUNE_NF4_FUSED
 #define SS_TUNE_NF4_FUSED 1
 #endif
