@@ -397,7 +397,10 @@ PYBIND11_MODULE(_native, m) {
   name_node<NF4Linear>("NF4LinearBackward");
   name_node<RowNorm>("RowNormBackward");
   name_node<QLoRA>("_QLoRAFusedBackward");
-  m.def("nf4_linear", &nf4_linear);
-  m.def("row_norm", &row_norm);
-  m.def("qlora", &qlora);
+  // Without the interpreter lock: a call may wait for room in the launch queue or for memory,
+  // and other threads run meanwhile, as they do during a ctypes call.
+  using Unlocked = pybind11::call_guard<pybind11::gil_scoped_release>;
+  m.def("nf4_linear", &nf4_linear, Unlocked());
+  m.def("row_norm", &row_norm, Unlocked());
+  m.def("qlora", &qlora, Unlocked());
 }

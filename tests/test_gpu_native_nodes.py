@@ -1,6 +1,10 @@
 """The native autograd nodes against the Python nodes they stand for: same kernels on the
 same operands, so outputs and gradients are bit-identical, and the same refusals."""
 
+import sys
+import threading
+import time
+
 import pytest
 import torch
 
@@ -8,6 +12,7 @@ from soupsuck_amd import _lib, lora
 from soupsuck_amd.bnb_compat import matmul_4bit, quantize_4bit
 from soupsuck_amd.kernels.add_rmsnorm import add_rms_norm
 from soupsuck_amd.kernels.rmsnorm import rms_norm
+from soupsuck_amd.native import nodes
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -123,3 +128,50 @@ def test_native_node_refuses_what_the_python_node_refuses(make):
     with pytest.raises((RuntimeError, ValueError)):
         torch.func.vmap(lambda x: fn(x, *[a.detach() for a in args[1:]]))(
             torch.stack([args[0].detach()] * 2))
+
+
+def _native_call(name):
+    """A call of one native entry point with no other Python code in it."""
+    native, x = nodes(), _randn(32768, 128)
+    if name == "row_norm":
+        w = _randn(128, seed=2)
+        return lambda: native.row_norm(x, None, w, 1e-6, False)
+    packed, state = _weight(192, 128)
+    second = state.state2
+    weight = (packed, state.absmax, second.absmax, second.code, state.offset, 192, 128)
+    if name == "nf4_linear":
+        return lambda: native.nf4_linear(x, *weight, None)
+    a, b = _randn(16, 128, seed=5), _randn(192, 16, seed=6)
+    stream = _lib.stream(x.device)
+    ws = lora._gemm_ws(32768, 192, 128, x.device, stream)[0]
+    rank_ws = lora._qlora_rank_ws(32768, 192, 128, x.device, stream)
+    return lambda: native.qlora(x, a, b, *weight, None, 2.0, None, ws, rank_ws)
+
+
+@pytest.mark.parametrize("name", ["nf4_linear", "row_norm", "qlora"])
+def test_other_threads_run_during_a_native_call(name):
+    """The entry points give up the interpreter lock: with a switch interval longer than the
+    test, another thread advances only where the calling one lets go of it."""
+    call = _native_call(name)
+    call()
+    turns, stop = [0], threading.Event()
+
+    def other():
+        while not stop.is_set():
+            turns[0] += 1
+            time.sleep(0)
+
+    thread = threading.Thread(target=other)
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(60.0)
+    try:
+        thread.start()          # start() waits for the thread's first turn
+        before, kept = turns[0], []
+        while turns[0] == before and len(kept) < 600:
+            kept.append(call())     # kept: freeing a tensor may give up the lock too
+        assert turns[0] > before
+    finally:
+        stop.set()
+        sys.setswitchinterval(interval)
+        thread.join()
+    torch.cuda.synchronize()
