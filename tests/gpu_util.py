@@ -1,11 +1,28 @@
 """Helpers shared by the GPU parity tests (host-side conversions only)."""
 
+import ctypes
 from types import SimpleNamespace
 
 import numpy as np
 import torch
 
 from oracle import nf4 as onf4
+from soupsuck_amd import _lib
+
+
+class _NtPlan(ctypes.Structure):
+    _fields_ = [("cfg", ctypes.c_int), ("splits", ctypes.c_int64), ("k_split", ctypes.c_int64)]
+
+
+def nt_plan(m, n, k, layout=0, split=True):
+    """(configuration, splits) that the dense kernels take for an M x N x K product (ss::nt_plan in
+    csrc/gemm_nt.hip; pure host code): layout bit 0 / 1 for a K-major A / B, split=False
+    without scratch."""
+    plan = _lib.load()._ZN2ss7nt_planElllim
+    plan.restype = _NtPlan
+    plan.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int, ctypes.c_size_t]
+    got = plan(m, n, k, layout, ctypes.c_size_t(-1).value if split else 0)
+    return got.cfg, got.splits
 
 
 def device_state(state, device):
