@@ -501,7 +501,7 @@ __global__ __launch_bounds__(C::kThreads, C::MINW) void gemm_nf4t_kernel(GemmPar
 #pragma unroll
     for (int j = 0; j < C::FN; ++j) acc[i][j] = float16v{};
   nf4k_mainloop<C, CD>(p, m0, n0, kbeg, klen, smem, acc);
-  nt_epilogue<C, CT, EPI>(p, m0, n0, acc, smem, split);
+  nt_epilogue<C, CT, EPI, sizeof(smem)>(p, m0, n0, acc, smem, split);
 }
 
 template <class C, int CD, int CT, int EPI>
@@ -526,7 +526,7 @@ __global__ __launch_bounds__(C::kThreads, C::MINW) void gemm_nf4_kernel(GemmPara
 #pragma unroll
     for (int j = 0; j < C::FN; ++j) acc[i][j] = float16v{};
   nf4_mainloop<C, CD>(p, m0, n0, kbeg, klen, smem, acc);
-  nt_epilogue<C, CT, EPI>(p, m0, n0, acc, smem, split);
+  nt_epilogue<C, CT, EPI, sizeof(smem)>(p, m0, n0, acc, smem, split);
 }
 
 // Configurations (1 and 2 in nf4_plan).

@@ -393,7 +393,7 @@ __global__ __launch_bounds__(C::kThreads, C::MINW) void gemm_nt_kernel(GemmParam
   } else {
     nt_mainloop_pp<C, L>(p, m0, n0, kbeg, klen, smem, acc);
   }
-  nt_epilogue<C, CT, EPI>(p, m0, n0, acc, smem, split);
+  nt_epilogue<C, CT, EPI, sizeof(smem)>(p, m0, n0, acc, smem, split);
 }
 
 // Split-K reduction: out[row][col] = epilogue(sum over splits s = 0.. of

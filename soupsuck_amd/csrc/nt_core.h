@@ -454,7 +454,7 @@ __device__ __forceinline__ void nt_epilogue_staged(const GemmParams& p, int64_t 
 // `smem`: the kernel's LDS, SMEM bytes, which the staged epilogues use.
 template <class C, int CT, int EPI, int SMEM>
 __device__ __forceinline__ void nt_epilogue(const GemmParams& p, int64_t m0, int64_t n0,
-                                            const NtAcc<C>& acc, unsigned char (&smem)[SMEM],
+                                            const NtAcc<C>& acc, unsigned char* smem,
                                             int64_t split = 0) {
   if constexpr (EPI == EPI_GLU) {
     if constexpr (GluStage<C>::kOk) {
@@ -468,7 +468,9 @@ __device__ __forceinline__ void nt_epilogue(const GemmParams& p, int64_t m0, int
     return;
   }
   if constexpr (CT == SS_F16 && EPI != EPI_PARTIAL && GluStage<C>::kOk) {
-    if (p.c_vec) {
+    // (The test of smem, never null here, keeps the register allocation of the 256-wide tiles
+    // out of scratch: without it the 256x256 ones spill 45 to 96 registers.)
+    if (p.c_vec && smem) {
       nt_epilogue_staged<C, EPI, SMEM>(p, m0, n0, acc, smem);
       return;
     }

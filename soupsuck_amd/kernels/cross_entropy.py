@@ -20,14 +20,14 @@ differentiable, ValueError before launch) and its numerics (:1-43):
             scattered to all rows (ss_ce_finalize_dx).  Ignored rows get zero
             gradient whatever the upstream value.
 
-Extension (``weight_grad=True``, asked for by BASELINE configs[3]): the
+Extension (``weight_grad=True``): the
 reference only accepts a frozen head (ValueError "frozen"); here the head
 gradient dW_c = dz'^T . h is also produced, from a second fp16 copy dz' of the
 derivative scaled by one global gain max_r |g_r| / 1024 (a per-row gain cannot
 be factored out of a sum over rows).
 
 Kept logits: when the fp16 logits [N, V] fit KEEP_LOGITS_BUDGET (1 GiB; 251 MB
-at configs[3]) and a backward may run, the forward's products write into one
+at 826 x 151936) and a backward may run, the forward's products write into one
 [N, V] buffer and the backward reads the logits from there (rows picked through
 the labelled-row indices) instead of recomputing h . W_c^T: one product per
 chunk fewer.  The forward's product then spans the whole vocabulary of an fp16 head
@@ -35,7 +35,7 @@ chunk fewer.  The forward's product then spans the whole vocabulary of an fp16 h
 its pieces are those of a chunk-by-chunk forward, so the
 outputs are the same bits.  The backward's
 steps span as many chunks as DERIVATIVE_BUDGET holds of dz and dz' (the whole
-vocabulary at configs[3]): one derivative launch and two long products.  Above
+vocabulary at 826 x 151936): one derivative launch and two long products.  Above
 KEEP_LOGITS_BUDGET the backward recomputes, as the reference does, one [rows,
 chunk] tile at a time.
 
@@ -54,7 +54,7 @@ from .. import _lib
 from ..contract import FLOAT_DTYPES, Rule, enforce, on_one_cuda_device
 from .nf4_gemm import gemm_f16
 
-MAX_CHUNK = 8192            # BASELINE configs[3]'s vocabulary chunk
+MAX_CHUNK = 8192            # vocabulary columns of a chunk at most
 TILE_BUDGET = 64 << 20      # bytes of one fp16 [rows, chunk] logits tile
 # Bytes of fp16 logits [rows, V] the forward may keep for the backward, which
 # then reads them instead of recomputing each chunk's product (the same bits:

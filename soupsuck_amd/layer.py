@@ -104,7 +104,7 @@ class DecoderLayer:
     kernels: RMSNorm -> q/k/v QLoRA projections -> joint q/k RoPE -> causal attention
     within each packed row -> o projection -> residual add + RMSNorm -> gate/up
     projections -> SwiGLU -> down projection -> residual add.  Forward then backward
-    of the whole layer from an upstream gradient (the north star's full-layer time).
+    of the whole layer from an upstream gradient (the full-layer time that the benchmark reports).
     The seven projections are ``QLoRALayer``'s; norm weights ~ 1 + N(0, 0.1) fp16;
     RoPE angles are Qwen2's (theta 1e6) at each token's position within its row."""
 
