@@ -15,8 +15,8 @@ assert_close(rtol=2e-3, atol=2e-3) on the fp16 output plus relative L2 <= 1e-3.
 
 Beyond EXP-002's calibrated reductions (K <= 8960), ``no_worse_than_reference``
 compares the errors of a result and of the reference's own decode-then-dense
-path against the exact-weight product (the north star's "no worse than the
-reference's own error").
+path against the exact-weight product ("no worse than the reference's
+own error").
 
 Pins: the float64 product is numpy's matmul (a library routine); tests plant a
 transposed operand and a dropped bias in the oracle on tiny shapes and check
@@ -69,7 +69,7 @@ def no_worse_than_reference(actual, exact, reference, slack=SLACK):
     product of the fp16-decoded weight with the output rounded to fp16.  Both the
     largest element error and the relative L2 error of ``actual`` against
     ``exact`` may exceed the reference's by at most the factor ``slack``.  This is
-    the north star's "no worse than the reference's own error", for reductions
+    the bar "no worse than the reference's own error", for reductions
     longer than EXP-002 calibrated its fixed 2e-3 element tolerance on (K <= 8960):
     there the rounding of each decoded weight alone moves the decoded-weight
     product by more than 2e-3 (the deviation grows as sqrt(K)).

@@ -7,10 +7,10 @@
 //
 // Operand layouts, configurations and the epilogue: nt_core.h.
 //
-// Two main loops: NtStream (4 waves, 64-deep stages; every configuration that nt_plan
-// weighs) and the ping-pong loop of eight waves with 32-deep stages, which stays ahead
-// where A lies K-major (the cross-entropy's dW, 151936 x 1536 x 576: 320 us against 336
-// us on 128x128 stream tiles).
+// Two main loops: NtStream (4 waves, 64-deep stages) and the ping-pong loop of eight
+// waves with 32-deep stages, which stays ahead for short K (nt_plan) and where A lies
+// K-major (the cross-entropy's dW, 151936 x 1536 x 576: 320 us against 336 us on 128x128
+// stream tiles).
 //
 // The DMA is issued from inline asm.  The compiler does not know which LDS
 // buffer an outstanding LDS DMA writes, and would wait for all of them
@@ -614,6 +614,8 @@ int dispatch_nt(const GemmParams& p, int cfg, int64_t splits, hipStream_t stream
     case 5: return launch_nt<Nt256x160, CT, EPI>(p, splits, stream);
     case 6: return launch_nt<Nt256x192, CT, EPI>(p, splits, stream);
     case 7: return launch_nt<Nt256, CT, EPI>(p, splits, stream);
+    case 8:
+      if constexpr (EPI != EPI_PARTIAL) return launch_nt<NtPingPong, CT, EPI>(p, splits, stream);
     default: return SS_ERR_UNSUPPORTED;
   }
 }
@@ -644,26 +646,36 @@ static size_t nt_split_bytes(int64_t m, int64_t n, int64_t splits) {
 
 // Configuration and split-K plan for an M x N x K product: the cheapest by a cost model
 // of the time a launch takes,
-//   start + q (tile + stages (stage + load f)),   q = ceil(workgroups / CUs),
-// with a configuration's start, epilogue and 64-deep stage times in us and f the busy
-// share of the CUs (with all of them busy the clock falls), plus a split's reduce.
-// The constants are least-squares fits to 156 products of this kernel measured on
-// MI355X (M 260 .. 16384 at the Qwen2.5 1.5B and 7B projection shapes, every
-// configuration and up to 5 splits); the model's choice takes 1.02 times the best
-// measured one on average, 1.10 at the 95th percentile.  Against the former rules and
-// kernels (32-deep stages, tiles by thresholds on the tile count), us before -> after:
-// 990 x 1536 x 1536 16.5 -> 9.7, 990 x 256 x 1536 11.9 -> 6.7, 990 x 8960 x 1536 35.4 ->
-// 29.2, 826 x 8960 x 1536 32.9 -> 25.7, 990 x 1536 x 8960 43.7 -> 38.5, 990 x 3584 x 3584
-// 44.2 -> 29.5, 2048 x 3584 x 3584 62.2 -> 50.3, 16384 x 18944 x 3584 1898 -> 1771.
+//   start + q tile + stages (q stage + ceil(q / 2) pair + w load),
+//   w = workgroups / CUs, q = ceil(w),
+// with a configuration's start, epilogue and 64-deep stage times in us (load: the part that
+// grows with the busy share of the chip, clock and caches; pair: the part that two
+// workgroups on a CU overlap), plus a split's reduce.  A long K (8192 or more walked by more
+// than one workgroup per CU in turn; 3584 on 64-column tiles) adds `drift` to a stage: the
+// workgroups fall out of step along K and share less of the caches (16384 x 3584 x 18944 on
+// 256x192 tiles 2097 us, 1923 on 128x256).  K is split only where the tiles leave CUs idle.
+// The constants are least-squares fits to 4500 products of these kernels measured on
+// MI355X (M 260 .. 16384, N 256 .. 18944, K 64 .. 18944, every configuration, and up to 8
+// splits of the long K); the model's choice takes 1.005 times the best measured one on
+// average, 1.03 at the 95th percentile.  Against the kernels before the 64-deep stages
+// (thresholds on the tile count), us before -> now: 990 x 1536 x 1536 16.5 -> 10.5, 990 x 8960 x
+// 1536 37 -> 31, 990 x 1536 x 8960 45 -> 42, 2048 x 3584 x 3584 63 -> 50, 16384 x 18944 x 3584
+// 1898 -> 1771.  The ping-pong tile stays ahead for short K, where it fills the chip: 3500
+// x 3584 x 512 19.4 us (128x256 stream tiles 22.4), 2700 x 4864 x 896 29.3 (31.4), 1350 x 8960 x
+// 1536 43.3 (44.8), 16384 x 8960 x 256 116 (131).
 struct TileCost {
   int cfg, bm, bn;
-  float start, tile, stage, load;
+  float start, tile, stage, pair, load, drift;
 };
 constexpr TileCost kTileCosts[] = {
-    {1, 64, 64, 3.6f, 0.0f, 0.151f, 0.043f},     {2, 128, 64, 3.8f, 0.0f, 0.227f, 0.094f},
-    {3, 128, 128, 1.6f, 2.6f, 0.281f, 0.196f},   {4, 128, 256, 0.0f, 6.4f, 0.460f, 0.322f},
-    {5, 256, 160, 0.0f, 7.7f, 0.553f, 0.393f},   {6, 256, 192, 0.0f, 7.6f, 0.711f, 0.468f},
-    {7, 256, 256, 0.0f, 13.1f, 0.896f, 0.532f},
+    {1, 64, 64, 3.47f, 0.44f, 0.037f, 0.139f, 0.055f, 0.023f},
+    {2, 128, 64, 3.47f, 0.99f, 0.225f, 0.0f, 0.043f, 0.032f},
+    {3, 128, 128, 2.68f, 2.79f, 0.279f, 0.0f, 0.165f, 0.047f},
+    {4, 128, 256, 2.52f, 4.85f, 0.451f, 0.0f, 0.338f, 0.069f},
+    {5, 256, 160, 2.71f, 6.18f, 0.534f, 0.0f, 0.407f, 0.088f},
+    {6, 256, 192, 2.23f, 6.85f, 0.712f, 0.0f, 0.404f, 0.184f},
+    {7, 256, 256, 2.53f, 11.76f, 0.848f, 0.0f, 0.575f, 0.130f},
+    {8, 256, 256, 1.69f, 6.70f, 0.846f, 0.0f, 0.738f, 0.222f},
 };
 
 // layout: bit 0 / 1 for K-major A / B (GemmParams::a_t, b_t).  scratch: what the planes of
@@ -684,15 +696,20 @@ NtPlan nt_plan(int64_t m, int64_t n, int64_t k, int layout, size_t scratch) {
   for (const TileCost& c : kTileCosts) {
     if (layout && c.cfg != 1 && c.cfg != 3 && c.cfg != 4) continue;
     const int64_t tiles = cdiv(m, c.bm) * cdiv(n, c.bn);
-    for (int64_t s = 1; s <= most; ++s) {
+    const int64_t splits = c.cfg == 8 || tiles > cus ? 1 : most;  // 8: short K only
+    for (int64_t s = 1; s <= splits; ++s) {
       const int64_t k_split = cdiv(cdiv(k, s), 64) * 64;
       if (cdiv(k, k_split) != s) continue;
       if (s > 1 && nt_split_bytes(m, n, s) > scratch) break;
-      const int64_t q = cdiv(tiles * s, cus);
-      const float f = (float)(tiles * s) / (float)(q * cus);
+      const float w = (float)(tiles * s) / (float)cus;
+      const int64_t turns = cdiv(tiles * s, cus);
+      const float q = (float)turns, pairs = (float)cdiv(turns, 2);
+      const bool drifts = c.bn == 64 ? k >= 3584 : k >= 8192 && turns > 1;
+      const float stage = c.stage + (drifts ? c.drift : 0.0f);
       const float stages = (float)(k_split / 64);
-      float us = c.start + (float)q * (c.tile + stages * (c.stage + c.load * f));
-      if (s > 1) us += 5.4f + ((float)s * 1.01f + 0.29f) * (float)m * (float)n * 1e-6f;
+      float us = c.start + q * c.tile + stages * (q * stage + pairs * c.pair + c.load * w);
+      // (a split has to win by 3 %: ties go to the plan without planes)
+      if (s > 1) us = 1.03f * (us + 4.6f + (float)s * 1.05f * (float)m * (float)n * 1e-6f);
       if (best == 0.0f || us < best) {
         best = us;
         plan = NtPlan{c.cfg, s, k_split};

@@ -15,9 +15,13 @@ def test_tile_tests_reach_every_configuration():
     for t, n, k, forward, backward in QLORA:
         assert (nt_plan(t, n, k), nt_plan(t, k, n)) == (forward, backward), (t, n, k)
     tiles = {(c, s > 1) for *_, c, s in TILES}
-    assert {(c, False) for c in range(1, 8)} | {(c, True) for c in range(3, 8)} <= tiles
-    assert {(c, s > 1) for *_, c, s in K_MAJOR} >= {(3, False), (4, False), (8, False), (3, True),
-                                                   (4, True)}
+    every = {(c, False) for c in range(1, 9)} | {(c, True) for c in range(1, 8)}
+    assert every <= tiles
+    assert {(c, s > 1) for *_, c, s in K_MAJOR} == {(1, True), (3, False), (3, True), (4, False),
+                                                   (8, False)}
+    wide = {(c, False) for c in range(2, 9)} | {(2, True), (3, True), (5, True)}
+    for side in (3, 4):
+        assert wide <= {(row[side][0], row[side][1] > 1) for row in QLORA}
 
 
 @pytest.mark.parametrize("m,n,k", [(990, 1536, 8960), (300, 3584, 18944), (523, 1536, 151936)])

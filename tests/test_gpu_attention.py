@@ -5,7 +5,7 @@ flash attention): against the float64 oracle (oracle/attention.py) of the same
 fp16 inputs, the output within atol = rtol = 2e-3 elementwise and relative L2
 <= 2e-3; the base-2 lse within 1e-3 of lse / ln 2; gradients dQ, dK, dV within
 relative L2 1e-2 (fp16 outputs of sums over up to ~400 keys).  Cases: the
-configs[1] batch (4 rows, lengths uniform in [80, 400], seed 0, T = 990) with
+layer batch (4 rows, lengths uniform in [80, 400], seed 0, T = 990) with
 Qwen2.5-1.5B's 12 q heads and 2 kv heads; ragged rows of length 1 .. 130
 (block edges 64 / 65 / 128 / 129); no GQA and 8:1 GQA; transposed projection
 views as inputs; two calls bit-identical.

@@ -6,7 +6,7 @@ matmuls, Qwen2's RMSNorm / rotate-half RoPE / SwiGLU formulas and causal
 softmax attention within each packed row, all in float32 on the GPU, with
 autograd for the gradients.  Bar: output, input gradient and every LoRA A / B
 gradient within relative L2 2e-2 (a chain of ten fp16-rounded ops against
-fp32), and the output of two runs bit-identical.  configs[1] batch: 4 rows,
+fp32), and the output of two runs bit-identical.  Batch: 4 rows,
 lengths uniform in [80, 400] (seed 0), T = 990.
 """
 

@@ -5,7 +5,7 @@ experiments/reports/EXP-002.md:60-76): assert_close(rtol=2e-3, atol=2e-3) on
 the fp16 output against the float64 product of the bit-exact decoded weight
 (oracle.gemm), finite output, relative L2 <= 1e-3.  Shapes: the reference's
 EXP-002 table (W 1536x1536, 256x1536, 8960x1536, 1536x8960 at M = 800 and
-2048), configs[0] (gate 8960x1536, X [1024, 1536]), small-T rows (1, 16, 128),
+2048), the 1.5B gate projection (8960x1536, X [1024, 1536]), small-T rows (1, 16, 128),
 ragged sizes, the large-T decode-first path, and K % 64 != 0 (dense path).
 """
 
@@ -43,7 +43,7 @@ def check(actual, expected, what):
 
 
 @pytest.mark.parametrize("t,n,k", [
-    (1024, 8960, 1536),                                   # configs[0]
+    (1024, 8960, 1536),                                   # the 1.5B gate projection
     (800, 1536, 1536), (800, 256, 1536), (800, 8960, 1536), (800, 1536, 8960),
     (2048, 256, 1536),
     (1, 1536, 1536), (16, 8960, 1536), (128, 256, 1536), (37, 320, 128), (130, 192, 64),
@@ -161,9 +161,9 @@ def test_streaming_dx_small_t(device, t, n, k):
     check(out, ogemm.linear_dx(dy, w) + base.astype(np.float64), f"stream dx accumulate t={t}")
 
 
-# Decode-first products at the configs[1] layer shapes (T = 990: 256x256
-# tiles for 990x8960x1536, split-K 128x128 for the long-K 990x1536x8960,
-# 64x64 split-K for the narrow 990x256x1536), ragged T and N; split-K sums in
+# Decode-first products at the 1.5B layer shapes (T = 990: 256x160 tiles for
+# 990x8960x1536, 128x64 for 990x1536x1536, 128x256 split in five for the long-K
+# 990x1536x8960, 64x64 for the narrow 990x256x1536), ragged T and N; split-K sums in
 # split order, so two calls give the same bits; accumulation (beta = 1).
 @pytest.mark.parametrize("t,n,k", [
     (990, 8960, 1536), (990, 1536, 1536), (990, 1536, 8960), (990, 256, 1536),
@@ -256,14 +256,14 @@ def test_dense_gemm_layouts(device, a_trans, b_trans, out_dtype, m, n, k):
                                    rtol=1e-5, atol=2e-4)
 
 
-@pytest.mark.parametrize("m,n,k", [(4100, 4128, 96),    # 256x256 tiles, ragged M and N
-                                   (1000, 2000, 1536),  # 128x128 tiles
+@pytest.mark.parametrize("m,n,k", [(4100, 4128, 96),    # K % 64 != 0: the general kernel
+                                   (1000, 2000, 1536),  # 128x64 tiles
                                    (100, 300, 64),      # 64x64 tiles
-                                   (990, 1536, 8960)])  # long K (a gate/up dX shape)
+                                   (990, 1536, 8960)])  # long K (a gate/up dX shape), unsplit
 @pytest.mark.parametrize("out_dtype", [torch.float16, torch.float32])
 def test_dense_nt_pipeline_tiles(device, m, n, k, out_dtype):
-    """A [M,K] . B[N,K]^T with both operands K-contiguous and K % 32 == 0: the
-    direct-to-LDS pipelined kernel at each of its tile sizes, plus beta = 1."""
+    """A [M,K] . B[N,K]^T with both operands K-contiguous: the direct-to-LDS pipelined
+    kernel (K % 64 == 0; its tiles' edges: test_gpu_gemm_tiles.py), plus beta = 1."""
     rng = np.random.default_rng(m + n + k)
     a = rng.standard_normal((m, k)).astype(np.float16)
     bt = (rng.standard_normal((n, k)) * 0.05).astype(np.float16)
@@ -302,11 +302,11 @@ def test_dense_split_k(device, m, n, k):
     check(h, 0.25 * prod, f"split fp16 {m}x{n}x{k}")
 
 
-@pytest.mark.parametrize("t,n,k", [(990, 8960, 1536),   # 256x256 tiles, 4 M tiles
-                                   (1024, 8960, 1536),  # configs[0]
-                                   (800, 1536, 1536),   # 64x64 tiles
-                                   (300, 256, 1536),    # 64x64 tiles split over k
-                                   (990, 1536, 8960)])  # decode-first (long k)
+@pytest.mark.parametrize("t,n,k", [(990, 8960, 1536),   # 256x160 tiles, 4 M tiles
+                                   (1024, 8960, 1536),
+                                   (800, 1536, 1536),   # 128x64 tiles
+                                   (300, 256, 1536),    # 64x64 tiles
+                                   (990, 1536, 8960)])  # 128x256 tiles split in five
 def test_forward_bitwise_equals_decode_then_dense(device, t, n, k):
     """The NF4 forward (fused decode or decode-first, as dispatched) equals,
     bit for bit, the stand-alone decode followed by the dense NT GEMM with the
@@ -325,14 +325,14 @@ def test_forward_bitwise_equals_decode_then_dense(device, t, n, k):
 
 
 @pytest.mark.parametrize("m,n,k,split", [
-    (2048, 3584, 512, False),   # 128x256 tiles (8 waves)
-    (4096, 4096, 128, False),   # 256x256 tiles, ping-pong main loop
-    (1024, 2048, 256, False),   # 128x128 tiles
-    (1000, 2008, 320, False),   # 128x128 tiles, ragged M and N
+    (2048, 3584, 512, False),   # 128x256 tiles
+    (4096, 4096, 128, False),   # 256x256 tiles, ping-pong main loop (K-major A), else 64x64
+    (1024, 2048, 256, False),   # 64x64 tiles
+    (1000, 2008, 320, False),   # 64x64 tiles, ragged M and N
     (200, 136, 1024, False),    # 64x64 tiles
-    (200, 136, 1024, True),     # 64x64 tiles split over K
-    (990, 1536, 8960, True),    # 256x128 tiles split over K
-    (1536, 1024, 4096, True),   # 128x128 tiles split over K
+    (200, 136, 1024, True),     # 64x64 tiles with scratch that they do not need
+    (990, 1536, 8960, True),    # 128x256 tiles split over K
+    (1536, 1024, 4096, True),   # 128x128 tiles
     (8, 16, 64, False),         # one 64x64 tile, 8-wide chunks clamped at M / N
 ])
 @pytest.mark.parametrize("a_trans,b_trans", [(False, False), (True, False), (True, True)])

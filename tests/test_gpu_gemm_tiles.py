@@ -47,38 +47,44 @@ def test_skinny_rows(device, t, n, k):
 
 
 # m, n, k, scratch for a split, then the plan: configuration (1 .. 7 for 64x64, 128x64, 128x128,
-# 128x256, 256x160, 256x192, 256x256; 8 the ping-pong 256x256 of a K-major A) and splits.  Every
-# configuration with M and N past a tile edge, unsplit and split with a shorter last split, the
-# small ones also with one to four 64-deep stages (a stage ring longer than the work, equal,
-# longer work) and on grids wider than the chip.
+# 128x256, 256x160, 256x192, 256x256; 8 the ping-pong 256x256) and splits.  Every configuration
+# with M and N past a tile edge, unsplit and split with a shorter last split (8 is not split),
+# the small ones also with one to four 64-deep stages (a stage ring longer than the work,
+# equal, longer work) and on grids wider than the chip.
 TILES = [
     (1, 8, 64, False, 1, 1), (65, 72, 128, False, 1, 1), (257, 264, 192, False, 1, 1),
-    (129, 2064, 256, False, 1, 1), (1025, 8008, 64, False, 1, 1), (1000, 8960, 192, False, 2, 1),
-    (2049, 4104, 128, False, 2, 1), (4100, 6408, 64, False, 2, 1), (300, 520, 1600, True, 1, 1),
-    (827, 264, 4160, True, 1, 3), (513, 1544, 8256, True, 1, 1),
-    (578, 3376, 256, False, 3, 1), (1170, 5128, 384, False, 4, 1), (1669, 5424, 384, False, 5, 1),
-    (1950, 5128, 384, False, 6, 1), (2576, 5496, 576, False, 7, 1),
-    (287, 1096, 5568, True, 3, 8), (259, 3824, 6016, True, 4, 5), (386, 3192, 9024, True, 5, 6),
-    (1428, 1320, 11392, True, 6, 6), (775, 5168, 10240, True, 7, 3),
+    (129, 2064, 256, False, 1, 1), (1025, 8008, 64, False, 1, 1), (1000, 8960, 192, False, 5, 1),
+    (2049, 4104, 128, False, 1, 1), (4100, 6408, 64, False, 8, 1), (300, 520, 1600, True, 1, 1),
+    (827, 264, 4160, True, 2, 7), (513, 1544, 8256, True, 3, 3), (130, 5512, 256, False, 1, 1),
+    (201, 5960, 192, False, 2, 1), (642, 4440, 128, False, 3, 1), (1235, 5704, 128, False, 4, 1),
+    (1170, 5128, 384, False, 4, 1), (1665, 5480, 128, False, 5, 1), (1680, 4832, 256, False, 5, 1),
+    (1547, 5928, 192, False, 6, 1), (1950, 5128, 384, False, 6, 1),
+    (2564, 5456, 3008, False, 7, 1), (1732, 5848, 64, False, 8, 1), (2375, 6024, 64, False, 8, 1),
+    (2576, 5496, 576, False, 8, 1), (12, 32, 2624, True, 1, 5), (2872, 8, 6016, True, 2, 8),
+    (67, 4120, 4864, True, 3, 7), (134, 5544, 7488, True, 4, 5), (130, 5704, 11968, True, 5, 7),
+    (2494, 544, 12096, True, 6, 8), (1026, 4088, 11648, True, 7, 3),
 ]
 # m, n, k, K-major A, K-major B, configuration, splits
 K_MAJOR = [
-    (1096, 2736, 128, True, False, 3, 1), (2440, 2912, 256, True, False, 4, 1),
-    (1861, 3784, 256, False, True, 4, 1), (1864, 3784, 256, True, True, 4, 1),
-    (72, 2784, 4416, True, False, 3, 8), (68, 2784, 4416, False, True, 3, 8),
-    (136, 5536, 5056, True, True, 4, 5), (1832, 3856, 64, True, False, 8, 1),
-    (1832, 3856, 192, True, True, 8, 1),
+    (528, 5488, 128, True, False, 3, 1), (1480, 4768, 128, True, False, 4, 1),
+    (1480, 4768, 128, False, True, 4, 1), (1480, 4768, 128, True, True, 4, 1),
+    (72, 4584, 4160, True, False, 3, 6), (72, 4584, 4160, False, True, 3, 6),
+    (72, 4584, 4160, True, True, 3, 6), (16, 8, 3904, False, True, 1, 7),
+    (1288, 5400, 64, True, False, 8, 1), (1832, 3856, 192, True, True, 8, 1),
 ]
 # t, n, k of a QLoRA projection, then the plans of its forward (t x n x k, LoRA epilogue) and of
 # its dX (t x k x n, rank-16 epilogue)
 QLORA = [
-    (1672, 3648, 384, (4, 1), (1, 1)), (1284, 6016, 448, (5, 1), (1, 1)),
-    (1806, 5504, 384, (6, 1), (1, 1)), (2562, 5504, 576, (7, 1), (2, 1)),
-    (265, 1216, 5632, (3, 8), (1, 1)), (261, 3648, 6016, (4, 5), (1, 1)),
-    (642, 5504, 5312, (5, 2), (3, 1)),
-    (1220, 384, 4928, (1, 1), (4, 1)), (1289, 448, 6016, (1, 1), (5, 1)),
-    (1665, 384, 5888, (1, 1), (6, 1)), (2455, 576, 5760, (2, 1), (7, 1)),
-    (385, 5632, 832, (3, 1), (3, 8)), (658, 5248, 5504, (3, 1), (5, 2)),
+    (327, 4032, 192, (2, 1), (1, 7)), (534, 5568, 128, (3, 1), (1, 8)),
+    (1217, 5760, 128, (4, 1), (1, 6)), (2372, 3904, 128, (5, 1), (2, 6)),
+    (1567, 6016, 192, (6, 1), (2, 6)), (2314, 5696, 2624, (7, 1), (4, 1)),
+    (1948, 5312, 128, (8, 1), (2, 7)), (278, 832, 3136, (1, 1), (1, 1)),
+    (267, 1856, 5824, (3, 5), (1, 1)), (646, 5504, 5696, (5, 2), (5, 2)),
+    (324, 192, 4352, (1, 8), (2, 1)), (514, 128, 5696, (1, 8), (3, 1)),
+    (1409, 128, 5056, (1, 5), (4, 1)), (1665, 128, 5504, (2, 8), (5, 1)),
+    (1561, 192, 6016, (2, 6), (6, 1)), (2330, 2880, 5184, (4, 1), (7, 1)),
+    (2313, 128, 4480, (2, 6), (8, 1)), (273, 3328, 832, (2, 1), (2, 6)),
+    (258, 5824, 1856, (1, 1), (3, 5)), (652, 5696, 5504, (5, 2), (5, 2)),
 ]
 
 

@@ -108,7 +108,7 @@ def test_decoder_layer_graph_replay_matches_eager(device):
     attention, SwiGLU, residual adds) captured as one HIP graph, as bench.py times it:
     every replay, with unrelated eager work and synchronisations between replays,
     reproduces the eager step bit for bit -- output, input gradient and every LoRA
-    gradient -- on the configs[1] batch."""
+    gradient -- on a batch of T = 990."""
     from soupsuck_amd.layer import DecoderLayer
 
     lengths = [382, 242, 208, 158]

@@ -4,7 +4,7 @@
   unfused composition (ss_nf4_gemm_fwd or _dx, then ss_swiglu_fwd or _bwd,
   both pinned against the oracles in their own tests) at T values that take
   each GEMM path: streaming (T <= 32), skinny (33-128), fused NF4 (129-256),
-  decode-first + dense NT (larger T), at the configs[1] shapes
+  decode-first + dense NT (larger T), at the 1.5B shapes
   (gate/up 8960 x 1536, down 1536 x 8960).
 * fused_qwen2_mlp against the eager fp32 module on the decoded weights, with
   the reference's tolerance (solution/tests/test_mlp.py:12, 63-89): outputs
@@ -271,7 +271,7 @@ def test_patched_qwen2_mlp_routes_through_the_fused_node(device):
 
 
 def test_mlp_graph_replay_matches_eager(device):
-    """The frozen NF4 MLP node forward + backward at the configs[1] shapes (T = 990,
+    """The frozen NF4 MLP node forward + backward at the 1.5B shapes (T = 990,
     1536 -> 8960 -> 1536) captured as one HIP graph: every replay, with unrelated eager
     work between replays, reproduces the eager output and input gradient bit for bit."""
     torch.manual_seed(781)

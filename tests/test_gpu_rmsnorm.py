@@ -8,7 +8,7 @@ ignores); fp16 outputs also differ from it on at most 1/1000 entries, by at
 most two fp16 ulps (after the reference's half-store rule, :14-37: a flipped
 rounding of q, then of w q); dgamma within the same
 magnitude-scaled fp32 budget as the add-RMSNorm tests.  Cases: Qwen2.5-1.5B
-hidden 1536 at the configs[2] row counts, the reference's dtype grid, a 2-D
+hidden 1536 at 826 and 4096 rows, the reference's dtype grid, a 2-D
 row-strided input, zero rows.
 """
 

@@ -3,10 +3,10 @@
 add-RMSNorm bar (solution/tests/test_add_rmsnorm.py:10-11): the new residual
 s is bit-exact; y and the input gradients within fp32 1e-5 / fp16 2e-3
 (rtol = atol) of oracle/rmsnorm.py; dgamma within the magnitude-scaled fp32
-reduction budget of that test (:14-44).  Shapes: configs[2] (fp16 [T, 1536],
+reduction budget of that test (:14-44).  Shapes: hidden 1536 (fp16 [T, 1536],
 T in {826, 4096, 16384}, w = 1 + N(0, 0.1), eps 1e-6) and the reference's
 dtype-promotion grid at (2, 5, 1000).
-Unpad bar: bit-exact; configs[2] batch [4, 360, 1536] fp16 with lengths
+Unpad bar: bit-exact; a batch [4, 360, 1536] fp16 with lengths
 uniform in [80, 360].
 """
 

@@ -1,12 +1,12 @@
-"""GPU parity of the NF4 forward and dX at BASELINE configs[4] (Qwen2.5-7B shapes).
+"""GPU parity of the NF4 forward and dX at the Qwen2.5-7B projection shapes.
 
 Shapes, W [N, K]: q/o 3584x3584, k/v 512x3584, gate/up 18944x3584, down
 3584x18944; T in {1, 16, 128, 2048, 16384}; both directions, through the same
 C-ABI entry points (ss_nf4_gemm_fwd / ss_nf4_gemm_dx) and the same workspace
 sizing the benchmark sweep uses, so every dispatched path of the sweep is the
-one checked here: streaming (T <= 32), skinny / fused (T <= 256), decode-first
-256x256 8-wave tiles at N = 18944, and split-K with the long K = 18944 of the
-down projection.
+one checked here: streaming (T <= 32), skinny / fused (T <= 256), decode-first on
+128x256, 256x160 and 256x256 tiles, split over K only below T = 2048 (the split of
+a long K at larger ragged T: test_gpu_gemm_tiles.py).
 
 Weights: seeded N(0, 0.02) fp16 quantized on the GPU (ss_nf4_quantize).  The
 decoded weight is checked bit for bit against oracle/nf4.py on the first, a
@@ -21,7 +21,7 @@ reductions up to 8960; over the 18944-long reductions here (down forward,
 gate/up dX) the fp16 rounding of each decoded weight alone moves the
 decoded-weight product by more than 2e-3 (the reference's own
 decode-then-dense result misses the exact-weight product by ~4.4e-3).  There
-the bar is the north star's "no worse than the reference's own error": the
+the bar is "no worse than the reference's own error": the
 relative L2 bound of EXP-002 still holds, and the largest element error and
 the relative L2 error against the exact-weight product (oracle.nf4
 decode_exact) are at most 1.25x those of the reference's fp16 decode-then-dense

@@ -8,7 +8,7 @@ Cases follow the reference's use (solution/tests/test_mlp.py:63-89,
 solution/tests/test_precompile.py:258,402-406): fp16 projection outputs,
 fp32 outputs under autocast, fp16 saved gate/up with an fp32 upstream, 3-D
 inputs, widths not a multiple of 8, strided and transposed views, and the
-configs[1] MLP width (T = 990, I = 8960).
+1.5B MLP width (T = 990, I = 8960).
 """
 
 import numpy as np
