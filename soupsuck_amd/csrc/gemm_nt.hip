@@ -688,15 +688,21 @@ NtPlan nt_plan(int64_t m, int64_t n, int64_t k, int layout, size_t scratch) {
     plan.cfg = 8;
     return plan;
   }
-  // Splits: at least 512 deep; more than 8 only where each still has 8192.
-  int64_t most = k / 512 < 8 ? k / 512 : (k / 8192 > 8 ? k / 8192 : 8);
-  if (most > 16) most = 16;
+  // Splits: at least 512 deep; more than 8 only where each still has 4096.
+  int64_t most = k / 512 < 8 ? k / 512 : (k / 4096 > 8 ? k / 4096 : 8);
+  if (most > 64) most = 64;
   if (most < 1) most = 1;
   float best = 0.0f;
   for (const TileCost& c : kTileCosts) {
-    if (layout && c.cfg != 1 && c.cfg != 3 && c.cfg != 4) continue;
+    // K-major operands: the tiles of dispatch_nt_t, of them the ping-pong one where only B is
+    // K-major (the cross-entropy's dX over the vocabulary, 1500 x 1536 x 151936: 605 us in 7
+    // splits, 684 on 128x256 tiles; 3000 x 3584 x 151936 2761 and 3142), and not the 64-column
+    // one over a long K, whose short rows stream at half the rate (64 x 1536 x 151936: 139 us,
+    // 98 on 128x128 tiles in 21 splits).
+    if (layout && c.cfg != 1 && c.cfg != 3 && c.cfg != 4 && !(c.cfg == 8 && layout == 2)) continue;
+    if (layout && c.cfg == 1 && k >= 16384) continue;
     const int64_t tiles = cdiv(m, c.bm) * cdiv(n, c.bn);
-    const int64_t splits = c.cfg == 8 || tiles > cus ? 1 : most;  // 8: short K only
+    const int64_t splits = tiles > cus || (c.cfg == 8 && layout != 2) ? 1 : most;
     for (int64_t s = 1; s <= splits; ++s) {
       const int64_t k_split = cdiv(cdiv(k, s), 64) * 64;
       if (cdiv(k, k_split) != s) continue;
@@ -705,7 +711,11 @@ NtPlan nt_plan(int64_t m, int64_t n, int64_t k, int layout, size_t scratch) {
       const int64_t turns = cdiv(tiles * s, cus);
       const float q = (float)turns, pairs = (float)cdiv(turns, 2);
       const bool drifts = c.bn == 64 ? k >= 3584 : k >= 8192 && turns > 1;
-      const float stage = c.stage + (drifts ? c.drift : 0.0f);
+      float stage = c.stage + (drifts ? c.drift : 0.0f);
+      // (a long K of K-major operands slows the narrower tiles: 1500 x 896 x 151936 509 us on
+      // 128x128 tiles in 3 splits, 408 on 256x256 ones in 10; 2048 x 3584 x 151936 2038 us on
+      // 128x256 tiles, 1884 on 256x256 ones in 2)
+      if (layout && k >= 16384) stage += c.cfg == 3 ? 0.10f : c.cfg == 4 ? 0.06f : 0.0f;
       const float stages = (float)(k_split / 64);
       float us = c.start + q * c.tile + stages * (q * stage + pairs * c.pair + c.load * w);
       // (a split has to win by 3 %: ties go to the plan without planes)

@@ -18,7 +18,7 @@ def test_tile_tests_reach_every_configuration():
     every = {(c, False) for c in range(1, 9)} | {(c, True) for c in range(1, 8)}
     assert every <= tiles
     assert {(c, s > 1) for *_, c, s in K_MAJOR} == {(1, True), (3, False), (3, True), (4, False),
-                                                   (8, False)}
+                                                   (8, False), (8, True)}
     wide = {(c, False) for c in range(2, 9)} | {(2, True), (3, True), (5, True)}
     for side in (3, 4):
         assert wide <= {(row[side][0], row[side][1] > 1) for row in QLORA}

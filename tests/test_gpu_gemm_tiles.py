@@ -66,11 +66,12 @@ TILES = [
 ]
 # m, n, k, K-major A, K-major B, configuration, splits
 K_MAJOR = [
-    (528, 5488, 128, True, False, 3, 1), (1480, 4768, 128, True, False, 4, 1),
-    (1480, 4768, 128, False, True, 4, 1), (1480, 4768, 128, True, True, 4, 1),
-    (72, 4584, 4160, True, False, 3, 6), (72, 4584, 4160, False, True, 3, 6),
-    (72, 4584, 4160, True, True, 3, 6), (16, 8, 3904, False, True, 1, 7),
-    (1288, 5400, 64, True, False, 8, 1), (1832, 3856, 192, True, True, 8, 1),
+    (1205, 3208, 9536, False, True, 8, 3), (528, 5488, 128, True, False, 3, 1),
+    (1480, 4768, 128, True, False, 4, 1), (1480, 4768, 128, False, True, 4, 1),
+    (1480, 4768, 128, True, True, 4, 1), (72, 4584, 4160, True, False, 3, 6),
+    (72, 4584, 4160, False, True, 3, 6), (72, 4584, 4160, True, True, 3, 6),
+    (16, 8, 3904, False, True, 1, 7), (1288, 5400, 64, True, False, 8, 1),
+    (1832, 3856, 192, True, True, 8, 1),
 ]
 # t, n, k of a QLoRA projection, then the plans of its forward (t x n x k, LoRA epilogue) and of
 # its dX (t x k x n, rank-16 epilogue)
