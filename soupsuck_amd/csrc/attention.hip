@@ -724,7 +724,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void attn_bwd_dkdv_kernel(AttnArgs 
     round2(ds[k >> 2], k, p0 * dp[2 * k], p1 * dp[2 * k + 1]);
   };
   // S and dP - delta of 32 queries, [q][key = mykey]; then dV += P^T . dO and dK += dS^T .
-  // Q.  As in the forward, one half's products run over the other's element-wise step.
+  // Q.  Whole tiles run one half's products over the other's element-wise step (the forward
+  // and dQ have theirs in one piece between the products).
   auto compute = [&](int qt, const unsigned char* buf) {
     const unsigned char* sQ = buf;
     const unsigned char* sO = buf + kTileBytes;

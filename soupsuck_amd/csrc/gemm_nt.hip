@@ -828,8 +828,9 @@ int gemm_nt(const GemmParams& p0, int ct, int epi, hipStream_t stream, void* par
     }
     // The SwiGLU epilogue moves three more planes through the tile's waves: on the four
     // waves of the wide tiles it outlasts what their loop gains (frozen MLP at T = 990,
-    // 1536 x 8960, both activations in epilogues: 435 us on 256 x 160 tiles, 323 us so), so the
-    // eight waves of the ping-pong tile do it there, or 128 x 128 tiles where few would run.
+    // 1536 x 8960, both activations in epilogues: 435 us on 256 x 160 tiles, 326 us so; 302 us
+    // with kernels of their own), so the eight waves of the ping-pong tile do it there, or 128
+    // x 128 tiles where few would run.
     if (p.glu) {
       int cfg = plan.cfg;
       if (cfg > 3) cfg = cdiv(p.M, 256) * cdiv(p.N, 256) >= device_cu_count() / 2 ? 8 : 3;

@@ -115,12 +115,12 @@ def _state_args(packed, state):
 
 
 # Where the SwiGLU runs by default: its own HBM-bound kernels (False) or the
-# GEMM epilogues (True; bit-identical).  Measured on MI355X at the configs[1]
-# shapes (T = 990): alone, the down dX with the activation in its epilogue takes
-# 66-70 us against 54-59 + 17 us for the product and the kernel; inside the
-# whole MLP step the epilogue variant measured 398-414 us against 386-401 us in
-# the same runs (every output tile reaches its epilogue at once, so the extra
-# gate / up traffic there overlaps no MFMA work).  Callers choose per call with
+# GEMM epilogues (True; bit-identical).  MLP forward + backward on MI355X, us, own
+# kernels / epilogues: 1536 -> 8960 at T = 1 70 / 69, 64 116 / 114, 256 195 / 195, 400 215 / 212,
+# 990 302 / 326, 2048 488 / 539, 4096 855 / 915; 3584 -> 18944 at T = 1 109 / 106, 256 459 / 461,
+# 400 659 / 721, 990 1048 / 1179, 4096 3263 / 3290.  From a few hundred rows on every output
+# tile reaches its epilogue at once, so the extra gate / up traffic there overlaps no MFMA
+# work; below, the epilogues save one launch of two.  Callers choose per call with
 # ``fuse=``.
 GLU_IN_EPILOGUE = False
 

@@ -147,3 +147,24 @@ def test_reversed_token_axis(device, lengths, hq, hk):
 
     for got, want in zip(run(True), run(False)):
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("n,tail", [(2048, 2e-5), (2048, 1e-5), (100, 5e-5), (3000, 1e-6)])
+def test_dominating_key_with_subnormal_tail(device, n, tail):
+    """One key at P = 1 and n - 1 keys at P = tail, an fp16 subnormal (below 6.1e-5) that adds up
+    to percents of the mass: the P.V product and the sum that O is divided by must both
+    count it.  Bound on O: its own rounding, and a half step of the subnormal P (2^-25) for
+    every key in the product and in the sum."""
+    print(f"case dominating key n={n} tail={tail}", flush=True)
+    gen = torch.Generator().manual_seed(n)
+    q, k = torch.zeros((1, 2, n, 128)), torch.zeros((1, 1, n, 128))
+    q[..., 0] = 8.0
+    k[0, 0, 0, 0] = np.log(1 / tail) / 8 * 128 ** 0.5
+    v = torch.rand((1, 1, n, 128), generator=gen) + 1.0
+    v[:, :, 0] = -1.0
+    q, k, v = (a.half().to(device) for a in (q, k, v))
+    o = packed_causal_attention(q, k, v, (n,), 128 ** -0.5)
+    ref, _ = oattn.forward(_np(q), _np(k), _np(v), (n,), 128 ** -0.5)
+    err = np.abs(o[0].float().cpu().numpy().astype(np.float64) - ref).max()
+    bound = 2.0 ** -11 * max(1.0, np.abs(ref).max()) + n * 2.0 ** -25 * (2.0 + np.abs(ref).max())
+    assert err <= bound, f"{err:.3e} of {bound:.3e}"

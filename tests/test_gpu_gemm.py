@@ -304,7 +304,7 @@ def test_dense_split_k(device, m, n, k):
 
 @pytest.mark.parametrize("t,n,k", [(990, 8960, 1536),   # 256x160 tiles, 4 M tiles
                                    (1024, 8960, 1536),
-                                   (800, 1536, 1536),   # 128x64 tiles
+                                   (800, 1536, 1536),   # 64x64 tiles
                                    (300, 256, 1536),    # 64x64 tiles
                                    (990, 1536, 8960)])  # 128x256 tiles split in five
 def test_forward_bitwise_equals_decode_then_dense(device, t, n, k):
@@ -326,13 +326,13 @@ def test_forward_bitwise_equals_decode_then_dense(device, t, n, k):
 
 @pytest.mark.parametrize("m,n,k,split", [
     (2048, 3584, 512, False),   # 128x256 tiles
-    (4096, 4096, 128, False),   # 256x256 tiles, ping-pong main loop (K-major A), else 64x64
+    (4096, 4096, 128, False),   # 256x256 tiles, ping-pong main loop
     (1024, 2048, 256, False),   # 64x64 tiles
     (1000, 2008, 320, False),   # 64x64 tiles, ragged M and N
     (200, 136, 1024, False),    # 64x64 tiles
     (200, 136, 1024, True),     # 64x64 tiles with scratch that they do not need
     (990, 1536, 8960, True),    # 128x256 tiles split over K
-    (1536, 1024, 4096, True),   # 128x128 tiles
+    (1536, 1024, 4096, True),   # 128x64 tiles, K-major ones 64x64
     (8, 16, 64, False),         # one 64x64 tile, 8-wide chunks clamped at M / N
 ])
 @pytest.mark.parametrize("a_trans,b_trans", [(False, False), (True, False), (True, True)])
